@@ -44,6 +44,7 @@ constexpr int C_TOTAL = 16 + 4;
 struct BatchJob {
     CameraRec camera;
     long long work_base;
+    long long valid_base;  // pixels' samples (W * H * spp) of the jobs before it
     int W, H, ntx8, npix8;
     int spp, pad;
     uint64_t seed;
@@ -108,6 +109,11 @@ struct PathBufs {
     int njobs;
     int sort_threshold;    // bounces with fewer extension rays skip the material sort
     long long work0;
+    // slots of the pass that hold a pixel (the others pad 8x8 tiles), and how
+    // many such slots lie before the pass (batch: before work0; single render:
+    // in the tiles before pass_q0)
+    int pass_valid;
+    long long valid0;
 };
 
 // Shadow-queue entries carry the path slot in the low kSlotBits bits and the
@@ -159,6 +165,24 @@ __device__ __forceinline__ SlotInfo slot_info(const PathBufs &P, int i) {
     r.y = (tile / ntx8) * 8 + (w >> 3);
     r.valid = r.x < r.W && r.y < r.H;
     return r;
+}
+
+// Pixels of the 8x8-tiled index space before tiled pixel (x, y) of a W x H
+// image: whole tile rows, whole tiles of this row, rows and pixels within the
+// tile (the last tile row and column may be narrower than 8).
+__host__ __device__ inline long long tiled_rank(int x, int y, int W, int H) {
+    const int x0 = x & ~7, y0 = y & ~7;
+    const int tw = W - x0 < 8 ? W - x0 : 8, th = H - y0 < 8 ? H - y0 : 8;
+    return (long long)y0 * W + (long long)x0 * th + (y - y0) * tw + (x - x0);
+}
+// The same for a tiled pixel index q of any slot, padding included.
+__host__ __device__ inline long long tiled_rank_q(long long q, int ntx8, int W, int H) {
+    const long long tile = q >> 6;
+    const int w = int(q & 63), ty = int(tile / ntx8), tx = int(tile % ntx8);
+    if (8 * ty >= H) return (long long)W * H;
+    const int tw = W - 8 * tx < 8 ? W - 8 * tx : 8, th = H - 8 * ty < 8 ? H - 8 * ty : 8;
+    const int r = w >> 3, c = w & 7;
+    return 8ll * ty * W + 8ll * tx * th + (r < th ? r * tw + (c < tw ? c : tw) : th * tw);
 }
 
 // Counter resets folded into kernels that do not read those counters.
@@ -256,42 +280,36 @@ __global__ void k_fill_f64(double *p, size_t n) {
     for (; i < n; i += stride) p[i] = 0.0;
 }
 
-// compact = 0: every slot holds a valid pixel (W and H multiples of 8), so the
-// extension queue is the identity and needs no atomics.
-__global__ void k_raygen(DeviceScene S, PathBufs P, int compact) {
+// Camera rays of the pass.  The first extension queue lists the slots that
+// hold a pixel, in slot order: a slot's place in it has a closed form
+// (tiled_rank), so padded tiles cost no atomics (appending them with one
+// atomic per wave ran at 11 ns an atomic, all waves on one counter: 4.9 ms of
+// 28 for 19.5M paths at 637x479, where this takes 0.7 ms).
+__global__ void k_raygen(DeviceScene S, PathBufs P) {
     int n = P.pass_ns * P.pass_nq;
     int stride = gridDim.x * blockDim.x;
-    if (!compact && blockIdx.x == 0 && threadIdx.x == 0) P.ctr[C_EXT + 0] = n;
-    for (int base = blockIdx.x * blockDim.x; base < n; base += stride) {
-        int i = base + threadIdx.x;
-        SlotInfo si{};
-        bool valid = false;
-        if (i < n) {
-            si = slot_info(P, i);
-            valid = si.valid;
-        }
-        if (valid) {
-            uint64_t stream = si.stream();
-            uint64_t inc = pcg_inc(stream);
-            uint64_t st = pcg_init_state(stream, P.jobs ? P.jobs[si.job].seed : P.seed);
-            double r0 = pcg_double(st, inc), r1 = pcg_double(st, inc);
-            D3 o, d;
-            const CameraRec &cam = P.jobs ? P.jobs[si.job].camera : S.camera;
-            sample_primary(cam, (si.x + r0) / si.W, (si.y + r1) / si.H, o, d);
-            P.rng[i] = st;
-            P.ray_o[i] = make_float4(float(o.x), float(o.y), float(o.z), 0.0f);
-            P.ray_d[i] = make_float4(float(d.x), float(d.y), float(d.z), __builtin_huge_valf());
-            P.tp[i] = make_float4(1.f, 1.f, 1.f, 1.f);
-            P.prev[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            P.depth[i] = 0;
-        }
-        if (i < n) P.rad[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (compact) {
-            int k = wave_append(valid, &P.ctr[C_EXT + 0]);
-            if (k >= 0) P.extq0[k] = uint32_t(i);
-        } else if (i < n) {
-            P.extq0[i] = uint32_t(i);
-        }
+    if (blockIdx.x == 0 && threadIdx.x == 0) P.ctr[C_EXT + 0] = P.pass_valid;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+        P.rad[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        const SlotInfo si = slot_info(P, i);
+        if (!si.valid) continue;
+        uint64_t stream = si.stream();
+        uint64_t inc = pcg_inc(stream);
+        uint64_t st = pcg_init_state(stream, P.jobs ? P.jobs[si.job].seed : P.seed);
+        double r0 = pcg_double(st, inc), r1 = pcg_double(st, inc);
+        D3 o, d;
+        const CameraRec &cam = P.jobs ? P.jobs[si.job].camera : S.camera;
+        sample_primary(cam, (si.x + r0) / si.W, (si.y + r1) / si.H, o, d);
+        P.rng[i] = st;
+        P.ray_o[i] = make_float4(float(o.x), float(o.y), float(o.z), 0.0f);
+        P.ray_d[i] = make_float4(float(d.x), float(d.y), float(d.z), __builtin_huge_valf());
+        P.tp[i] = make_float4(1.f, 1.f, 1.f, 1.f);
+        P.prev[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        P.depth[i] = 0;
+        const long long rank = tiled_rank(si.x, si.y, si.W, si.H);
+        const long long k = P.jobs ? P.jobs[si.job].valid_base + (long long)si.s * si.W * si.H + rank - P.valid0
+                                   : (long long)(si.s - P.pass_s0) * (P.pass_valid / P.pass_ns) + rank - P.valid0;
+        P.extq0[k] = uint32_t(i);
     }
 }
 

@@ -1333,7 +1333,9 @@ void render_impl(Scene &sc, const ljx_render_options *o, const ljx_exec_options 
             passes++;
             tm.begin(3, ev);
             launch(k_reset_counters, 1, 64, s, P.ctr, 0, C_TOTAL);
-            launch(k_raygen, shade_grid, 256, s, S, P, (W % 8 || H % 8) ? 1 : 0);
+            P.valid0 = tiled_rank_q(q0, ntx8, W, H);
+            P.pass_valid = int(ns * (tiled_rank_q(q0 + nq, ntx8, W, H) - P.valid0));
+            launch(k_raygen, shade_grid, 256, s, S, P);
             launch(k_alive_clear, shade_grid, 256, s, P, ns * nq);
             if (vol) launch(k_vol_init, shade_grid, 256, s, S, P);
             if (recording)
@@ -1557,10 +1559,19 @@ void batch_impl(const ljx_batch_job *jobs, size_t njobs, const ljx_exec_options 
         std::vector<int> order;         // job indices, smallest work first
         std::vector<BatchJob> table;
         BatchJob *dtable = nullptr;
-        long long total = 0;
+        long long total = 0, valid = 0;
         int capacity = 0, block = 256;
     };
     std::vector<GroupPlan> plans(groups.size());
+    // slots with a pixel among the first w work items of a group
+    auto valid_before = [](const GroupPlan &gp, long long w) {
+        if (w >= gp.total) return gp.valid;
+        size_t j = 0;
+        while (j + 1 < gp.table.size() && gp.table[j + 1].work_base <= w) j++;
+        const BatchJob &b = gp.table[j];
+        const long long local = w - b.work_base;
+        return b.valid_base + local / b.npix8 * b.W * b.H + tiled_rank_q(local % b.npix8, b.ntx8, b.W, b.H);
+    };
     uint64_t total_samples = 0;
     for (size_t k = 0; k < groups.size(); k++) {
         GroupPlan &gp = plans[k];
@@ -1583,6 +1594,8 @@ void batch_impl(const ljx_batch_job *jobs, size_t njobs, const ljx_exec_options 
             b.work_base = gp.total;
             b.accum = static_cast<double *>(dmalloc(size_t(b.W) * b.H * 3 * sizeof(double)));
             b.out = J.rgb_out_device;
+            b.valid_base = gp.valid;
+            gp.valid += (long long)b.W * b.H * b.spp;
             gp.total += work(j);
             total_samples += uint64_t(b.W) * b.H * b.spp;
             gp.table.push_back(b);
@@ -1656,7 +1669,9 @@ void batch_impl(const ljx_batch_job *jobs, size_t njobs, const ljx_exec_options 
                 P.pass_nq = n;
                 passes++;
                 launch(k_reset_counters, 1, 64, cs, P.ctr, 0, C_TOTAL);
-                launch(k_raygen, sgrid, 256, cs, S, P, 1);
+                P.valid0 = valid_before(gp, w0);
+                P.pass_valid = int(valid_before(gp, w0 + n) - P.valid0);
+                launch(k_raygen, sgrid, 256, cs, S, P);
                 launch(k_alive_clear, sgrid, 256, cs, P, n);
                 if (vol) launch(k_vol_init, sgrid, 256, cs, S, P);
                 int cur = 0;
