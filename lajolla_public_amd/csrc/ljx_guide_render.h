@@ -59,11 +59,13 @@ __device__ __forceinline__ void guide_infer_body(DeviceScene S, PathBufs P, cons
     // path), one index space over their entries.  Paths in other buckets
     // never read their guide direction, so the network runs on guided
     // vertices only.
-    __shared__ int bstart[kNumBuckets + 1];
+    __shared__ int bstart[kNumBuckets + 1], obase[kNumBuckets];
     if (threadIdx.x == 0) {
-        int acc = 0;
+        int acc = 0, at = 0;
         for (int B = 0; B < kNumBuckets; B++) {
             bstart[B] = acc;
+            obase[B] = at;
+            at += P.ctr[C_BUCKET + B];
             const bool sel = B == kBucketAny || (B < kNumMatTypes && guidable(B) && ((P.guide_mask >> B) & 1u));
             if (sel) acc += P.ctr[C_BUCKET + B];
         }
@@ -75,7 +77,7 @@ __device__ __forceinline__ void guide_infer_body(DeviceScene S, PathBufs P, cons
         if (!guidable(B) || ((P.guide_mask >> B) & 1u)) continue;
         const int nb = P.ctr[C_BUCKET + B];
         for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nb; k += gridDim.x * blockDim.x)
-            P.gdir[P.bucket[size_t(B) * P.capacity + k]] = make_float4(0.f, 0.f, 0.f, -1.f);
+            P.gdir[P.order[bucket_start(P, B) + k]] = make_float4(0.f, 0.f, 0.f, -1.f);
     }
     load_lds(sfrag, ffrag, kFwdFrags * 64, sbias, fbias, kBiasFwd);  // ends with a barrier
     const int n = bstart[kNumBuckets];
@@ -87,7 +89,7 @@ __device__ __forceinline__ void guide_infer_body(DeviceScene S, PathBufs P, cons
         if (i < n) {
             int B = 0;
             while (i >= bstart[B + 1]) B++;
-            uint32_t pid = P.bucket[size_t(B) * P.capacity + (i - bstart[B])];
+            uint32_t pid = P.order[obase[B] + (i - bstart[B])];
             float4 h = P.hit[pid];
             int slot = __float_as_int(h.w);
             if (slot >= 0) {

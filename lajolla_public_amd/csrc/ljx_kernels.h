@@ -4,9 +4,9 @@
 // into stages that each run over a compacted SoA queue of path ids:
 //
 //   k_raygen      sample_primary + the two screen-jitter draws
-//   k_extend      closest-hit traversal, 64 rays per wave fetch; appends each
-//                 path to the bucket of the hit material's type (material
-//                 sort) or to MISS
+//   k_extend      closest-hit traversal, 64 rays per wave fetch; keys each
+//                 queue entry by the hit material's type or MISS
+//   k_sort_*      orders the queue's paths by key (material sort)
 //   k_shade<MT>   one kernel per material type: emission + MIS of the hit
 //                 reached by the previous BSDF sample, Russian roulette,
 //                 throughput update, then NEE (light pick, point, shadow ray
@@ -27,17 +27,21 @@
 namespace ljx {
 
 constexpr int kNumMatTypes = 9;
-constexpr int kBucketMiss = 9;
-constexpr int kBucketNoMat = 10;
-constexpr int kBucketAny = 11;  // unsorted hits (below the sort threshold), shaded by runtime dispatch
+constexpr int kBucketAny = 9;  // unsorted hits (below the sort threshold), shaded by runtime dispatch
+constexpr int kBucketMiss = 10;
+constexpr int kBucketNoMat = 11;
 constexpr int kNumBuckets = 12;
 // counter slots
 constexpr int C_EXT = 0;      // C_EXT + (0|1): extension queues
 constexpr int C_SH = 2;       // shadow queue
-constexpr int C_BUCKET = 4;   // C_BUCKET + bucket
-constexpr int C_XFETCH = 16;  // C_XFETCH + (0|1): rays taken from extension queue 0|1 by the traversal
+constexpr int C_BUCKET = 4;   // C_BUCKET + bucket: its paths
 constexpr int C_FLQ = 18;     // volumetric free-flight queue: its length, then (C_FLQ + 1) paths taken from it
 constexpr int C_TOTAL = 16 + 4;
+// ticket counters of the traversal launches (Feed): two sets, used in turn by
+// the bounces, of kFeeds counters a 128-byte line apart
+constexpr int kFeeds = 8, kFeedLine = 32;
+constexpr int C_FEED = 32;
+constexpr int C_ALLOC = C_FEED + 2 * kFeeds * kFeedLine;
 
 // One job of a batched render: its camera, image and place in the batch's
 // global work index space (sample-major over its 8x8-tiled pixel grid).
@@ -65,7 +69,9 @@ struct PathBufs {
     float4 *ray_d;    // direction, tfar
     float4 *hit;      // t, u, v, slot (int bits; -1: miss)
     uint32_t *extq0, *extq1;
-    uint32_t *bucket; // kNumBuckets * capacity
+    uint8_t *key;     // per extension-queue entry: its hit's bucket
+    uint32_t *order;  // the extension queue's paths by bucket, each bucket in queue order
+    int *sort_blk;    // per bucket, per kScanBlock queue entries: paths, then their exclusive prefix
     uint32_t *shq;
     float4 *sh_o, *sh_d, *sh_c;
     uint8_t *sh_occ;  // per shadow ray: 1 when occluded
@@ -187,8 +193,7 @@ __host__ __device__ inline long long tiled_rank_q(long long q, int ntx8, int W, 
 
 // Counter resets folded into kernels that do not read those counters.
 __global__ void k_reset_counters(int *ctr, int first, int count) {
-    int i = threadIdx.x;
-    if (i < count) ctr[first + i] = 0;
+    for (int i = threadIdx.x; i < count; i += blockDim.x) ctr[first + i] = 0;
 }
 
 // The next bounce's extension queue: the slots shading marked alive, in slot
@@ -235,13 +240,14 @@ __global__ __launch_bounds__(256) void k_alive_count(PathBufs P, int n) {
     block_excl_scan(c, total);
     if (threadIdx.x == 0) P.alive_blk[blockIdx.x] = total;
 }
-__global__ __launch_bounds__(1024) void k_alive_scan(PathBufs P, int nblk, int cur) {
-    // 1024 threads x 16 blocks each: nblk <= 16384 (n <= 2^26)
+// Exclusive scan in place of n <= 16384 counts by one block of 1,024 threads
+// x 16 counts; returns the total in the last thread.
+__device__ __forceinline__ int scan_blocks(int *blk, int n) {
     __shared__ int part[1024];
     const int b0 = threadIdx.x * 16;
     int v[16], sum = 0;
     for (int k = 0; k < 16; k++) {
-        v[k] = b0 + k < nblk ? P.alive_blk[b0 + k] : 0;
+        v[k] = b0 + k < n ? blk[b0 + k] : 0;
         sum += v[k];
     }
     part[threadIdx.x] = sum;
@@ -254,10 +260,14 @@ __global__ __launch_bounds__(1024) void k_alive_scan(PathBufs P, int nblk, int c
     }
     int run = part[threadIdx.x] - sum;
     for (int k = 0; k < 16; k++) {
-        if (b0 + k < nblk) P.alive_blk[b0 + k] = run;
+        if (b0 + k < n) blk[b0 + k] = run;
         run += v[k];
     }
-    if (threadIdx.x == 1023) P.ctr[C_EXT + (cur ^ 1)] = part[1023];
+    return part[threadIdx.x];
+}
+__global__ __launch_bounds__(1024) void k_alive_scan(PathBufs P, int nblk, int cur) {
+    const int total = scan_blocks(P.alive_blk, nblk);
+    if (threadIdx.x == 1023) P.ctr[C_EXT + (cur ^ 1)] = total;
 }
 __global__ __launch_bounds__(256) void k_alive_scatter(PathBufs P, int n, int cur) {
     uint32_t *next = cur ? P.extq0 : P.extq1;
@@ -272,6 +282,93 @@ __global__ __launch_bounds__(256) void k_alive_scatter(PathBufs P, int n, int cu
             if ((w[j >> 2] >> (8 * (j & 3))) & 0xffu) next[k++] = uint32_t(s0 + j);
         *reinterpret_cast<uint4 *>(P.alive + s0) = make_uint4(0, 0, 0, 0);
     }
+}
+
+// The material sort of a bounce: a stable counting sort of the extension
+// queue's n entries by the keys k_extend wrote.  Appending each path to its
+// bucket's queue inside the traversal costs one atomic instruction per wave
+// on a counter line that every wave of the chip shares; such instructions run
+// one every 11.3 ns whatever their lanes, so 67M paths spent 12 ms there
+// (with Feed's counters: closest hits of a 1,048,576-path Cornell render 1.40
+// -> 0.34 ms, of the 1080p 64-sample terrain 70.4 -> 56.8 ms; the sort adds
+// 0.14 and 1.3 ms).
+// Three launches: counts per kScanBlock entries and bucket, their exclusive
+// scans (one block per bucket, which also sets the bucket's length), and the
+// scatter.  Buckets end up in queue order, so their paths' state stays near
+// coalesced.
+constexpr int kSortRows = kScanBlock / 256;  // a wave's 1,024 entries: 16 rows of 64
+// Wave-level ranks of a wave's rows of keys: rank[r] is the entry's place
+// among the wave's entries of its key; lane b returns the count of key b.
+__device__ __forceinline__ int sort_ranks(const int (&key)[kSortRows], int (&rank)[kSortRows]) {
+    const int lane = __lane_id();
+    int cnt = 0;
+#pragma unroll
+    for (int r = 0; r < kSortRows; r++) {
+        uint64_t pending = __ballot(key[r] >= 0);
+        rank[r] = 0;
+        while (pending) {
+            const int k = __builtin_amdgcn_readlane(key[r], __ffsll((unsigned long long)pending) - 1);
+            const uint64_t m = __ballot(key[r] == k);
+            const int before = __builtin_amdgcn_readlane(cnt, k);
+            if (key[r] == k)
+                rank[r] = before + int(__builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo(uint32_t(m), 0)));
+            if (lane == k) cnt += __popcll(m);
+            pending &= ~m;
+        }
+    }
+    return cnt;
+}
+__device__ __forceinline__ int sort_load(const PathBufs &P, int n, int (&key)[kSortRows]) {
+    const int i0 = blockIdx.x * kScanBlock + (threadIdx.x >> 6) * (64 * kSortRows) + (threadIdx.x & 63);
+#pragma unroll
+    for (int r = 0; r < kSortRows; r++) key[r] = i0 + 64 * r < n ? P.key[i0 + 64 * r] : -1;
+    return i0;
+}
+__global__ __launch_bounds__(256) void k_sort_count(PathBufs P, int cur, int nblk) {
+    __shared__ int wcnt[4][kNumBuckets];
+    const int n = P.ctr[C_EXT + cur];
+    if (blockIdx.x * kScanBlock >= n) return;
+    int key[kSortRows], rank[kSortRows];
+    sort_load(P, n, key);
+    const int cnt = sort_ranks(key, rank), lane = threadIdx.x & 63;
+    if (lane < kNumBuckets) wcnt[threadIdx.x >> 6][lane] = cnt;
+    __syncthreads();
+    const int b = threadIdx.x;
+    if (b < kNumBuckets) P.sort_blk[size_t(b) * nblk + blockIdx.x] = wcnt[0][b] + wcnt[1][b] + wcnt[2][b] + wcnt[3][b];
+}
+__global__ __launch_bounds__(1024) void k_sort_scan(PathBufs P, int cur, int nblk) {
+    // 1024 threads x 16 blocks each: at most 16384 blocks (n <= 2^26)
+    const int live = (P.ctr[C_EXT + cur] + kScanBlock - 1) / kScanBlock;
+    const int total = scan_blocks(P.sort_blk + size_t(blockIdx.x) * nblk, live);
+    if (threadIdx.x == 1023) P.ctr[C_BUCKET + blockIdx.x] = total;
+}
+// Where bucket b starts in P.order.
+__device__ __forceinline__ int bucket_start(const PathBufs &P, int b) {
+    int s = 0;
+    for (int k = 0; k < b; k++) s += P.ctr[C_BUCKET + k];
+    return s;
+}
+__global__ __launch_bounds__(256) void k_sort_scatter(PathBufs P, int cur, int nblk) {
+    __shared__ int wcnt[4][kNumBuckets], place[4][kNumBuckets];
+    const int n = P.ctr[C_EXT + cur];
+    if (blockIdx.x * kScanBlock >= n) return;
+    const uint32_t *q = cur ? P.extq1 : P.extq0;
+    int key[kSortRows], rank[kSortRows];
+    const int i0 = sort_load(P, n, key);
+    const int cnt = sort_ranks(key, rank), lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (lane < kNumBuckets) wcnt[w][lane] = cnt;
+    __syncthreads();
+    if (threadIdx.x < 4 * kNumBuckets) {
+        const int ww = threadIdx.x / kNumBuckets, b = threadIdx.x % kNumBuckets;
+        int at = bucket_start(P, b) + P.sort_blk[size_t(b) * nblk + blockIdx.x];
+        for (int k = 0; k < ww; k++) at += wcnt[k][b];
+        place[ww][b] = at;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortRows; r++)
+        if (key[r] >= 0) P.order[place[w][key[r]] + rank[r]] = q[i0 + 64 * r];
 }
 
 __global__ void k_fill_f64(double *p, size_t n) {
@@ -313,17 +410,56 @@ __global__ void k_raygen(DeviceScene S, PathBufs P) {
     }
 }
 
-// Closest-hit traversal of the extension queue.  A wave takes 64 rays at a
-// time with one atomic and walks them until the last one ends, so waves that
-// drew short rays take more and the launch's tail stays short; each hit's
-// distance is refined while its triangle is in cache, and the wave appends
-// its paths to the buckets of the materials they hit (the material sort)
-// with one atomic per bucket.  (Refilling lanes as their rays end, as
-// k_shadow does, measured slower here: the refill points run the finishing
-// work divergently and scatter the bucket order that shading reads.)
-// The fetch counter of a launch starts at zero: k_reset_counters clears
-// every counter at a pass's start and each launch clears the one the next
-// launch uses.
+// Hands a launch's n queue entries to its waves, 64 at a time, so that waves
+// that drew short work take more and the launch's tail stays short.  Each
+// wave's first chunk is its own by its number; after that it takes tickets.
+// A ticket is one atomic by the whole wave, and those on one cache line run
+// one every 11.3 ns on the whole chip (2,048 blocks took 12 ms of tickets for
+// 67M rays from a single counter), so blocks draw from kFeeds counters on
+// lines of their own, by block number modulo kFeeds, which is the XCD that
+// dispatch in turn places them on.  Feed f owns every kFeeds-th run of
+// kFeedRun chunks: an XCD's waves work on neighbouring entries, and every feed
+// sees all parts of the queue.
+constexpr int kFeedRun = 16;
+struct Feed {
+    int feeds, feed, waves, ticket;
+    int *counter;
+    bool more;  // chunks remain after every wave's first
+    __device__ __forceinline__ int chunk(int t) const {
+        return ((t / kFeedRun) * feeds + feed) * kFeedRun + t % kFeedRun;
+    }
+    // counters: a set of kFeeds zeroed counters kFeedLine apart.  Grids of
+    // fewer than kFeeds blocks use one feed.
+    __device__ __forceinline__ void start(int *counters, int n) {
+        const int wpb = blockDim.x >> 6;
+        feeds = int(gridDim.x) < kFeeds ? 1 : kFeeds;
+        feed = int(blockIdx.x) % feeds;
+        waves = (int(gridDim.x) + feeds - 1 - feed) / feeds * wpb;
+        ticket = __builtin_amdgcn_readfirstlane(int(blockIdx.x) / feeds * wpb + int(threadIdx.x >> 6));
+        counter = counters + feed * kFeedLine;
+        more = chunk(waves) < (n + 63) / 64;
+    }
+    // First entry of the wave's current chunk; at or past n: none is left.
+    __device__ __forceinline__ int base() const { return chunk(ticket) * 64; }
+    __device__ __forceinline__ void next(int n) {
+        if (!more) {
+            ticket = 1 << 20;  // past every queue (2^26 entries)
+            return;
+        }
+        int t = 0;
+        if (__lane_id() == 0) t = atomicAdd(counter, 1);
+        ticket = waves + __builtin_amdgcn_readfirstlane(t);
+    }
+};
+
+// Closest-hit traversal of the extension queue: a wave walks 64 rays (Feed)
+// until the last one ends; each hit's distance is refined while its triangle
+// is in cache, and each queue entry gets the key of the material it hit.
+// (Refilling lanes as their rays end, as k_shadow does, measured slower here:
+// the refill points run the finishing work divergently.)
+// The feed counters of a launch start at zero: k_reset_counters clears every
+// counter at a pass's start and each launch clears the set the next launch
+// uses.
 template <bool STATS, bool SPH>
 __device__ __forceinline__ int extend_finish(const DeviceScene &S, const PathBufs &P, uint32_t pid,
                                              const Tracer<false, STATS, SPH> &tr, bool sorted) {
@@ -342,9 +478,7 @@ __device__ __forceinline__ int extend_finish(const DeviceScene &S, const PathBuf
         P.hit[pid] = make_float4(0.f, 0.f, 0.f, __int_as_float(-1));
         bucket = kBucketMiss;
     }
-    // volumetric paths decide between medium and surface events after
-    // free-flight sampling: one queue
-    return P.volpath ? 0 : bucket;
+    return bucket;
 }
 
 // Triangle-only scenes: capped at 64 registers, eight waves per SIMD (the
@@ -358,36 +492,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? 1 : 8
     const bool sorted = n >= P.sort_threshold;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         P.ctr[C_SH] = 0;
-        P.ctr[C_XFETCH + (cur ^ 1)] = 0;
         atomicAdd(&P.stat[S_EXT_RAYS], (unsigned long long)n);
     }
-    int *fetch = &P.ctr[C_XFETCH + cur];
+    int *feeds = P.ctr + C_FEED;
+    if (blockIdx.x == 0 && threadIdx.x < kFeeds) feeds[((cur ^ 1) * kFeeds + threadIdx.x) * kFeedLine] = 0;
     const TraceScene ts{S.qnodes, S.prims, S.spheres};
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x;
     const int sstride = gridDim.x * blockDim.x;
     int *spill = P.spill + gtid;
     const int lane = __lane_id();
     uint32_t nn = 0, np = 0;
-    while (true) {
-        int base = 0;
-        if (lane == 0) base = atomicAdd(fetch, 64);
-        base = __shfl(base, 0);
-        if (base >= n) break;
+    Feed feed;
+    feed.start(feeds + cur * kFeeds * kFeedLine, n);
+    for (int base = feed.base(); base < n; feed.next(n), base = feed.base()) {
         const int i = base + lane;
-        int bucket = -1;
-        uint32_t pid = 0;
         if (i < n) {
-            pid = q[i];
+            const uint32_t pid = q[i];
             const float4 o = P.ray_o[pid], d = P.ray_d[pid];
             Tracer<false, STATS, SPH> tr;
             tr.start(o.x, o.y, o.z, d.x, d.y, d.z, o.w, d.w);
             if (S.num_nodes > 0)
                 while (!tr.step(ts, stack + threadIdx.x, blockDim.x, spill, sstride, nn, np)) {
                 }
-            bucket = extend_finish<STATS, SPH>(S, P, pid, tr, sorted);
+            const int bucket = extend_finish<STATS, SPH>(S, P, pid, tr, sorted);
+            if (!P.volpath) P.key[i] = uint8_t(bucket);
         }
-        const int k = wave_append_keyed(bucket, &P.ctr[C_BUCKET]);
-        if (bucket >= 0) P.bucket[size_t(bucket) * P.capacity + k] = pid;
     }
     if (STATS) {
         atomicAdd(&P.stat[S_NODES], (unsigned long long)nn);
@@ -572,7 +701,7 @@ template <int MT, bool SPH, bool GUIDE>
 __device__ __forceinline__ void shade_queue(const DeviceScene &S, const PathBufs &P, int cur) {
     constexpr int B = MT >= 0 ? MT : kBucketAny;
     int n = P.ctr[C_BUCKET + B];
-    const uint32_t *q = P.bucket + size_t(B) * P.capacity;
+    const uint32_t *q = P.order + bucket_start(P, B);
     int stride = gridDim.x * blockDim.x;
     for (int base = blockIdx.x * blockDim.x; base < n; base += stride) {
         int i = base + threadIdx.x;
@@ -615,7 +744,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // Escaped paths: environment emission with MIS (path_tracing.h:17-28, 284-302).
 __global__ __launch_bounds__(256) void k_miss(DeviceScene S, PathBufs P) {
     int n = P.ctr[C_BUCKET + kBucketMiss];
-    const uint32_t *q = P.bucket + size_t(kBucketMiss) * P.capacity;
+    const uint32_t *q = P.order + bucket_start(P, kBucketMiss);
     if (S.envmap_light_id < 0) return;
     const LightRec &env = S.lights[S.envmap_light_id];
     int stride = gridDim.x * blockDim.x;
@@ -670,7 +799,6 @@ __global__ __launch_bounds__(256) void k_shadow(DeviceScene S, PathBufs P) {
     const int n = P.ctr[C_SH];
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         atomicAdd(&P.stat[S_SH_RAYS], (unsigned long long)n);
-        for (int b = 0; b < kNumBuckets; b++) P.ctr[C_BUCKET + b] = 0;
     }
     const TraceScene ts{S.qnodes, S.prims, S.spheres};
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x;

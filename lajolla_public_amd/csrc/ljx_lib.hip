@@ -1027,7 +1027,8 @@ void ensure_ctx(Scene &sc, int capacity, int trace_grid) {
     P.hit = sc.alloc<float4>(C, rc->bufs);
     P.extq0 = sc.alloc<uint32_t>(C, rc->bufs);
     P.extq1 = sc.alloc<uint32_t>(C, rc->bufs);
-    P.bucket = sc.alloc<uint32_t>(C * kNumBuckets, rc->bufs);
+    P.key = sc.alloc<uint8_t>(C, rc->bufs);
+    P.order = sc.alloc<uint32_t>(C, rc->bufs);
     P.shq = sc.alloc<uint32_t>(C, rc->bufs);
     P.sh_o = sc.alloc<float4>(C, rc->bufs);
     P.sh_d = sc.alloc<float4>(C, rc->bufs);
@@ -1036,7 +1037,8 @@ void ensure_ctx(Scene &sc, int capacity, int trace_grid) {
     const size_t nblk = (C + kScanBlock - 1) / kScanBlock;
     P.alive = sc.alloc<uint8_t>(nblk * kScanBlock, rc->bufs);
     P.alive_blk = sc.alloc<int>(nblk, rc->bufs);
-    P.ctr = sc.alloc<int>(C_TOTAL, rc->bufs);
+    P.sort_blk = sc.alloc<int>(nblk * kNumBuckets, rc->bufs);
+    P.ctr = sc.alloc<int>(C_ALLOC, rc->bufs);
     P.stat = sc.alloc<unsigned long long>(S_NUM, rc->bufs);
     P.spill = sc.alloc<int>(size_t(rc->trace_grid) * 256 * sc.spill_entries, rc->bufs);
     P.accum = sc.alloc<double>(size_t(sc.width) * sc.height * 3, rc->bufs);
@@ -1133,6 +1135,15 @@ void build_ext_queue(PathBufs &P, int n, int cur, hipStream_t s) {
     launch(k_alive_count, nblk, 256, s, P, n);
     launch(k_alive_scan, 1, 1024, s, P, nblk, cur);
     launch(k_alive_scatter, nblk, 256, s, P, n, cur);
+}
+
+// The bucket order of the extension queue from the keys traversal left
+// (k_sort_*); n: the pass's slots, an upper bound of the queue's length.
+void sort_ext_queue(PathBufs &P, int n, int cur, hipStream_t s) {
+    const int nblk = (n + kScanBlock - 1) / kScanBlock;
+    launch(k_sort_count, nblk, 256, s, P, cur, nblk);
+    launch(k_sort_scan, kNumBuckets, 1024, s, P, cur, nblk);
+    launch(k_sort_scatter, nblk, 256, s, P, cur, nblk);
 }
 
 void trace_stage(Scene &sc, PathBufs &P, int cur, int grid, int sgrid, hipStream_t s, bool stats, bool shadow) {
@@ -1309,7 +1320,7 @@ void render_impl(Scene &sc, const ljx_render_options *o, const ljx_exec_options 
     hipEvent_t ev;
     tm.begin(3, ev);
     launch(k_fill_f64, 1024, 256, s, P.accum, size_t(W) * H * 3);
-    launch(k_reset_counters, 1, 64, s, P.ctr, 0, C_TOTAL);
+    launch(k_reset_counters, 1, 64, s, P.ctr, 0, C_ALLOC);
     hipLaunchKernelGGL(k_reset_stats, dim3(1), dim3(64), 0, s, P.stat);
     HIPX(hipGetLastError());
     tm.end(3, ev);
@@ -1332,7 +1343,7 @@ void render_impl(Scene &sc, const ljx_render_options *o, const ljx_exec_options 
             P.rec_stride = ns * nq;
             passes++;
             tm.begin(3, ev);
-            launch(k_reset_counters, 1, 64, s, P.ctr, 0, C_TOTAL);
+            launch(k_reset_counters, 1, 64, s, P.ctr, 0, C_ALLOC);
             P.valid0 = tiled_rank_q(q0, ntx8, W, H);
             P.pass_valid = int(ns * (tiled_rank_q(q0 + nq, ntx8, W, H) - P.valid0));
             launch(k_raygen, shade_grid, 256, s, S, P);
@@ -1353,6 +1364,11 @@ void render_impl(Scene &sc, const ljx_render_options *o, const ljx_exec_options 
                 tm.begin(0, ev);
                 trace_stage(sc, P, cur, tgrid, shade_grid, s, stats_on, false);
                 tm.end(0, ev);
+                if (!vol) {
+                    tm.begin(2, ev);
+                    sort_ext_queue(P, ns * nq, cur, s);
+                    tm.end(2, ev);
+                }
                 if (guided) {
                     tm.begin(4, ev);
                     guide_infer(sc, P, cur, guide_grid, s, *net);
@@ -1668,7 +1684,7 @@ void batch_impl(const ljx_batch_job *jobs, size_t njobs, const ljx_exec_options 
                 P.pass_q0 = 0;
                 P.pass_nq = n;
                 passes++;
-                launch(k_reset_counters, 1, 64, cs, P.ctr, 0, C_TOTAL);
+                launch(k_reset_counters, 1, 64, cs, P.ctr, 0, C_ALLOC);
                 P.valid0 = valid_before(gp, w0);
                 P.pass_valid = int(valid_before(gp, w0 + n) - P.valid0);
                 launch(k_raygen, sgrid, 256, cs, S, P);
@@ -1677,6 +1693,7 @@ void batch_impl(const ljx_batch_job *jobs, size_t njobs, const ljx_exec_options 
                 int cur = 0;
                 for (int b = 0; b < std::max(P.max_depth, 1); b++) {
                     trace_stage(sc, P, cur, tgrid, sgrid, cs, false, false);
+                    if (!vol) sort_ext_queue(P, n, cur, cs);
                     if (vol) vol_shade_all(S, P, cur, sgrid, cs, sc.has_spheres, (sc.mat_types_present & ~7u) == 0);
                     else shade_all(sc, P, cur, sgrid, cs, false, gp.block);
                     build_ext_queue(P, n, cur, cs);

@@ -156,10 +156,11 @@ __device__ __forceinline__ double hit_distance(const DeviceScene &S, float4 h, D
 // (the order does not matter: each path's flight uses its own stream).  Each
 // block of 1,024 threads appends with one atomic per round (a wave per
 // atomic contended on the one counter).
-__global__ __launch_bounds__(1024) void k_vol_flight_queue(PathBufs P) {
+__global__ __launch_bounds__(1024) void k_vol_flight_queue(PathBufs P, int cur) {
     __shared__ int wcount[16];
     __shared__ int bbase;
-    const int n = P.ctr[C_BUCKET + 0];
+    const int n = P.ctr[C_EXT + cur];
+    const uint32_t *q = cur ? P.extq1 : P.extq0;
     const int stride = gridDim.x * blockDim.x;
     const int w = threadIdx.x >> 6;
     for (int base = blockIdx.x * blockDim.x; base < n; base += stride) {
@@ -167,7 +168,7 @@ __global__ __launch_bounds__(1024) void k_vol_flight_queue(PathBufs P) {
         uint32_t pid = 0;
         bool in_medium = false;
         if (i < n) {
-            pid = P.bucket[i];
+            pid = q[i];
             in_medium = P.medium[pid] >= 0;
         }
         const uint64_t mask = __ballot(in_medium);
@@ -426,8 +427,10 @@ __device__ __forceinline__ void vol_shade(const DeviceScene &S, const PathBufs &
 
 template <bool SPH, int DMT>
 __global__ __launch_bounds__(256) void k_vol_shade(DeviceScene S, PathBufs P, int cur) {
-    int n = P.ctr[C_BUCKET + 0];
-    const uint32_t *q = P.bucket;
+    // paths decide between medium and surface events after free-flight
+    // sampling, so they are not sorted: the extension queue as it is
+    int n = P.ctr[C_EXT + cur];
+    const uint32_t *q = cur ? P.extq1 : P.extq0;
     int stride = gridDim.x * blockDim.x;
     for (int base = blockIdx.x * blockDim.x; base < n; base += stride) {
         int i = base + threadIdx.x;
@@ -522,9 +525,6 @@ template <bool STATS, bool SPH>
 __global__ __launch_bounds__(256) void k_vol_shadow(DeviceScene S, PathBufs P) {
     __shared__ int stack[kStackLds * 256];
     int n = P.ctr[C_SH];
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        for (int b = 0; b < kNumBuckets; b++) P.ctr[C_BUCKET + b] = 0;
-    }
     int gtid = blockIdx.x * blockDim.x + threadIdx.x;
     int stride = gridDim.x * blockDim.x;
     int *spill = P.spill + gtid;
@@ -669,7 +669,7 @@ inline void vol_launch_check() {
 inline void vol_shade_all(const DeviceScene &S, PathBufs &P, int cur, int grid, hipStream_t s, bool sph, bool basic) {
     if (P.vol_flight) {
         hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, P.ctr, C_FLQ, 2);
-        hipLaunchKernelGGL(k_vol_flight_queue, dim3(std::max(1, grid / 4)), dim3(1024), 0, s, P);
+        hipLaunchKernelGGL(k_vol_flight_queue, dim3(std::max(1, grid / 4)), dim3(1024), 0, s, P, cur);
         if (sph) hipLaunchKernelGGL(k_vol_flight<true>, dim3(grid), dim3(256), 0, s, S, P);
         else hipLaunchKernelGGL(k_vol_flight<false>, dim3(grid), dim3(256), 0, s, S, P);
         vol_launch_check();

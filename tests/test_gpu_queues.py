@@ -50,3 +50,25 @@ def test_ragged_batch_in_any_pass(cap):
         one = api.Scene(d).render(samples_per_pixel=j["spp"], max_depth=4, seed=j["seed"])
         # the same samples, added in another order in FP64 and rounded once to FP32
         assert np.allclose(img, one, rtol=2e-6, atol=1e-9)
+
+
+@pytest.mark.parametrize("w,h,spp", [(31, 33, 1), (64, 16, 1), (64, 64, 1), (64, 65, 2), (320, 257, 1), (640, 480, 2)])
+def test_material_sort_at_block_edges(w, h, spp):
+    """Several material types and misses, queues from under one wave's 1,024 entries to past the traversal's first
+    tickets: the image does not depend on the traversal grid (who takes which chunk) nor on the pass."""
+    desc = scenes.textured_showcase(seed=5)
+    desc.camera = scenes.orbit_camera(desc, np.random.default_rng(3), w, h, yaw_deg=4, pitch_deg=2, dist_range=(1, 1))
+    desc.options.update(samples_per_pixel=spp, max_depth=5)
+    sc = api.Scene(desc)
+    img, st = sc.render(stats=True)
+    assert np.isfinite(img).all() and img.mean() > 0
+    for bpc, cap in ((1, 0), (3, 0), (8, 1 << 12), (1, 1000)):
+        if cap and w * h * spp > 100000:
+            continue
+        got, sg = sc.render(options=scenes.render_options(**desc.options), stats=True,
+                            exec_options=api.exec_options(max_paths_in_flight=cap, trace_blocks_per_cu=bpc))
+        assert (sg["extension_rays"], sg["shadow_rays"]) == (st["extension_rays"], st["shadow_rays"])
+        if cap == 0:
+            assert np.array_equal(img, got), (bpc, cap)
+        else:  # a pixel's samples added in other groups in FP64, rounded once to FP32
+            assert np.allclose(img, got, rtol=2e-6, atol=1e-9), (bpc, cap)
