@@ -33,15 +33,17 @@ constexpr int kBucketNoMat = 11;
 constexpr int kNumBuckets = 12;
 // counter slots
 constexpr int C_EXT = 0;      // C_EXT + (0|1): extension queues
-constexpr int C_SH = 2;       // shadow queue
+constexpr int C_SH = 2;       // shadow queue (volumetric)
 constexpr int C_BUCKET = 4;   // C_BUCKET + bucket: its paths
 constexpr int C_FLQ = 18;     // volumetric free-flight queue: its length, then (C_FLQ + 1) paths taken from it
 constexpr int C_TOTAL = 16 + 4;
-// ticket counters of the traversal launches (Feed): two sets, used in turn by
-// the bounces, of kFeeds counters a 128-byte line apart
-constexpr int kFeeds = 8, kFeedLine = 32;
+// ticket counters (Feed), in sets of kFeeds a 128-byte line apart: two for
+// the closest-hit launches, used in turn by the bounces, and one each for the
+// bounce's other launches
+constexpr int kFeeds = 8, kFeedLine = 32, kFeedSet = kFeeds * kFeedLine;
 constexpr int C_FEED = 32;
-constexpr int C_ALLOC = C_FEED + 2 * kFeeds * kFeedLine;
+constexpr int C_FEED_SHADOW = C_FEED + 2 * kFeedSet;
+constexpr int C_ALLOC = C_FEED + 3 * kFeedSet;
 
 // One job of a batched render: its camera, image and place in the batch's
 // global work index space (sample-major over its 8x8-tiled pixel grid).
@@ -72,9 +74,10 @@ struct PathBufs {
     uint8_t *key;     // per extension-queue entry: its hit's bucket
     uint32_t *order;  // the extension queue's paths by bucket, each bucket in queue order
     int *sort_blk;    // per bucket, per kScanBlock queue entries: paths, then their exclusive prefix
-    uint32_t *shq;
     float4 *sh_o, *sh_d, *sh_c;
-    uint8_t *sh_occ;  // per shadow ray: 1 when occluded
+    uint8_t *sh_occ;  // per shadow ray: 0 unoccluded (or not traced yet), 1 occluded, kShNone where there is none
+    unsigned long long *wave_stat;  // per wave of the traversal grid: shadow rays traced
+    int waves;                      // its length
     uint8_t *alive;   // per path slot: 1 when shading gave it another ray (cleared as the queue is built)
     int *alive_blk;   // per kScanBlock slots: live paths, then their exclusive prefix
     // volumetric path state
@@ -122,6 +125,9 @@ struct PathBufs {
     long long valid0;
 };
 
+// A surface vertex's shadow ray is written at its path's place in P.order;
+// places without one carry this mark in sh_occ.
+constexpr uint8_t kShNone = 3;
 // Shadow-queue entries carry the path slot in the low kSlotBits bits and the
 // vertex index in the rest (clamped there: only the guiding record, a few
 // vertices deep, reads it).
@@ -495,7 +501,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? 1 : 8
         atomicAdd(&P.stat[S_EXT_RAYS], (unsigned long long)n);
     }
     int *feeds = P.ctr + C_FEED;
-    if (blockIdx.x == 0 && threadIdx.x < kFeeds) feeds[((cur ^ 1) * kFeeds + threadIdx.x) * kFeedLine] = 0;
+    if (blockIdx.x == 0 && threadIdx.x < kFeeds) {
+        feeds[(cur ^ 1) * kFeedSet + threadIdx.x * kFeedLine] = 0;
+        P.ctr[C_FEED_SHADOW + threadIdx.x * kFeedLine] = 0;
+    }
     const TraceScene ts{S.qnodes, S.prims, S.spheres};
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x;
     const int sstride = gridDim.x * blockDim.x;
@@ -503,7 +512,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? 1 : 8
     const int lane = __lane_id();
     uint32_t nn = 0, np = 0;
     Feed feed;
-    feed.start(feeds + cur * kFeeds * kFeedLine, n);
+    feed.start(feeds + cur * kFeedSet, n);
     for (int base = feed.base(); base < n; feed.next(n), base = feed.base()) {
         const int i = base + lane;
         if (i < n) {
@@ -700,22 +709,19 @@ __device__ __forceinline__ void shade_surface(const DeviceScene &S, const PathBu
 template <int MT, bool SPH, bool GUIDE>
 __device__ __forceinline__ void shade_queue(const DeviceScene &S, const PathBufs &P, int cur) {
     constexpr int B = MT >= 0 ? MT : kBucketAny;
-    int n = P.ctr[C_BUCKET + B];
-    const uint32_t *q = P.order + bucket_start(P, B);
-    int stride = gridDim.x * blockDim.x;
-    for (int base = blockIdx.x * blockDim.x; base < n; base += stride) {
-        int i = base + threadIdx.x;
+    const int n = P.ctr[C_BUCKET + B], start = bucket_start(P, B);
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const int j = start + i;
+        const uint32_t pid = P.order[j];
         bool pe = false, ps = false;
         float4 so, sd, sc;
-        uint32_t pid = 0;
-        if (i < n) {
-            pid = q[i];
-            shade_surface<MT, SPH, GUIDE>(S, P, pid, pe, ps, so, sd, sc);
-        }
+        shade_surface<MT, SPH, GUIDE>(S, P, pid, pe, ps, so, sd, sc);
         if (pe) P.alive[pid] = 1;
-        int j = wave_append(ps, &P.ctr[C_SH]);
-        if (j >= 0) {
-            P.shq[j] = pid;
+        // the shadow ray takes its path's place in the order: appending it to
+        // a queue costs an atomic per wave on one counter (11.3 ns each, one
+        // after the other: 38 of 122 ms for the 1080p terrain at 64 samples)
+        P.sh_occ[j] = ps ? uint8_t(0) : kShNone;
+        if (ps) {
             P.sh_o[j] = so;
             P.sh_d[j] = sd;
             P.sh_c[j] = sc;
@@ -786,20 +792,50 @@ __global__ __launch_bounds__(256) void k_miss(DeviceScene S, PathBufs P) {
     }
 }
 
-// Any-hit traversal of the shadow queue, rays assigned to lanes by a grid
-// stride; writes whether each is occluded (k_shadow_resolve adds the
+// A wave's current range of a queue it takes lane by lane (k_shadow): chunks
+// of 64 entries from a Feed.
+struct FeedRange {
+    Feed feed;
+    int cursor, end, n;
+    bool done;  // the feed has no more chunks
+    __device__ __forceinline__ void open() {
+        cursor = feed.base();
+        done = cursor >= n;
+        if (done) cursor = n;
+        end = min(n, cursor + 64);
+    }
+    __device__ __forceinline__ void start(int *counters, int n_) {
+        n = n_;
+        feed.start(counters, n);
+        open();
+    }
+    // A new chunk once the current one is used up.
+    __device__ __forceinline__ void refill() {
+        if (cursor < end || done) return;
+        feed.next(n);
+        open();
+    }
+    // The entry of the k-th of the wave's asking lanes (asked of them in
+    // total), or -1.
+    __device__ __forceinline__ int take(int k, int asked) {
+        const int i = cursor + k < end ? cursor + k : -1;
+        cursor = min(end, cursor + asked);
+        return i;
+    }
+};
+
+// Any-hit traversal of the bounce's shadow rays (the places of P.order up to
+// the misses); writes whether each is occluded (k_shadow_resolve adds the
 // contributions).  A lane whose ray ended takes its next one as soon as
 // kShadowRefill lanes of its wave are idle, instead of waiting for the
 // wave's longest ray (3.6% faster on the 1080p large-mesh render than
-// starting the lanes' rays together).
+// starting the lanes' rays together); places without a ray leave their lane
+// idle until the next such turn.
 constexpr int kShadowRefill = 16;
 template <bool STATS, bool SPH>
 __global__ __launch_bounds__(256) void k_shadow(DeviceScene S, PathBufs P) {
     __shared__ int stack[kStackLds * 256];
-    const int n = P.ctr[C_SH];
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        atomicAdd(&P.stat[S_SH_RAYS], (unsigned long long)n);
-    }
+    const int n = bucket_start(P, kBucketMiss);
     const TraceScene ts{S.qnodes, S.prims, S.spheres};
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x;
     const int stride = gridDim.x * blockDim.x;
@@ -807,30 +843,31 @@ __global__ __launch_bounds__(256) void k_shadow(DeviceScene S, PathBufs P) {
     uint32_t nn = 0, np = 0;
     Tracer<true, STATS, SPH> tr;
     bool busy = false, fin = false;
-    // each wave walks its own contiguous share of the queue (neighbouring
-    // rays come from neighbouring paths), its idle lanes taking the next
-    // rays of it in order
-    const int nwaves = stride >> 6;
-    const int per = (n + nwaves - 1) / nwaves;
-    int cursor = (gtid >> 6) * per;
-    const int end = min(n, cursor + per);
-    int i = 0;
+    FeedRange range;
+    range.start(P.ctr + C_FEED_SHADOW, n);
+    int i = 0, rays = 0;
     while (true) {
         const uint64_t idle = __ballot(!busy);
         const int nidle = __popcll(idle);
         if (nidle >= kShadowRefill) {
             if (fin) P.sh_occ[i] = tr.found ? 1 : 0;
             fin = false;
-            const int k = cursor + int(__builtin_amdgcn_mbcnt_hi(uint32_t(idle >> 32),
-                                                                 __builtin_amdgcn_mbcnt_lo(uint32_t(idle), 0)));
-            if (!busy && k < end) {
+            range.refill();
+            const int k = range.take(int(__builtin_amdgcn_mbcnt_hi(uint32_t(idle >> 32),
+                                                                   __builtin_amdgcn_mbcnt_lo(uint32_t(idle), 0))),
+                                     nidle);
+            if (!busy && k >= 0 && P.sh_occ[k] != kShNone) {
                 i = k;
                 const float4 o = P.sh_o[i], d = P.sh_d[i];
                 tr.start(o.x, o.y, o.z, d.x, d.y, d.z, o.w, d.w);
                 busy = true;
             }
-            cursor = min(end, cursor + nidle);
-            if (__ballot(busy) == 0) break;
+            const int now = __popcll(__ballot(busy));
+            rays += now - (64 - nidle);
+            if (now == 0) {
+                if (range.done) break;
+                continue;
+            }
         }
         if (busy) {
             if (S.num_nodes == 0 || tr.step(ts, stack + threadIdx.x, blockDim.x, spill, stride, nn, np)) {
@@ -839,6 +876,8 @@ __global__ __launch_bounds__(256) void k_shadow(DeviceScene S, PathBufs P) {
             }
         }
     }
+    // (one slot per wave: an atomic per wave on a shared total takes 93 us a launch)
+    if (__lane_id() == 0) P.wave_stat[gtid >> 6] += (unsigned long long)rays;
     if (STATS) {
         atomicAdd(&P.stat[S_SH_NODES], (unsigned long long)nn);
         atomicAdd(&P.stat[S_SH_PRIMS], (unsigned long long)np);
@@ -849,9 +888,9 @@ __global__ __launch_bounds__(256) void k_shadow(DeviceScene S, PathBufs P) {
 // to its path (and to the recorded radiance of its vertex when guiding
 // records the pass).
 __global__ __launch_bounds__(256) void k_shadow_resolve(PathBufs P) {
-    const int n = P.ctr[C_SH];
+    const int n = bucket_start(P, kBucketMiss);
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        if (P.sh_occ[i]) continue;
+        if (P.sh_occ[i] != 0) continue;
         const float4 c = P.sh_c[i];
         const uint32_t bits = uint32_t(__float_as_int(c.w));
         const uint32_t pid = bits & kSlotMask;
@@ -864,6 +903,19 @@ __global__ __launch_bounds__(256) void k_shadow_resolve(PathBufs P) {
             *rc = make_float4(o.x + c.x, o.y + c.y, o.z + c.z, 0.f);
         }
     }
+}
+
+// Render statistics: cleared at a render's start, and the waves' shadow rays
+// added up at its end.
+__global__ __launch_bounds__(1024) void k_reset_stats(PathBufs P) {
+    if (threadIdx.x < S_NUM) P.stat[threadIdx.x] = 0;
+    for (int i = threadIdx.x; i < P.waves; i += 1024) P.wave_stat[i] = 0;
+}
+__global__ __launch_bounds__(1024) void k_sum_stats(PathBufs P) {
+    unsigned long long s = 0;
+    for (int i = threadIdx.x; i < P.waves; i += 1024) s += P.wave_stat[i];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if ((threadIdx.x & 63) == 0) atomicAdd(&P.stat[S_SH_RAYS], s);
 }
 
 // render.cpp:89-94 (path) and :136-145 (volpath drops non-finite samples).

@@ -1029,7 +1029,6 @@ void ensure_ctx(Scene &sc, int capacity, int trace_grid) {
     P.extq1 = sc.alloc<uint32_t>(C, rc->bufs);
     P.key = sc.alloc<uint8_t>(C, rc->bufs);
     P.order = sc.alloc<uint32_t>(C, rc->bufs);
-    P.shq = sc.alloc<uint32_t>(C, rc->bufs);
     P.sh_o = sc.alloc<float4>(C, rc->bufs);
     P.sh_d = sc.alloc<float4>(C, rc->bufs);
     P.sh_c = sc.alloc<float4>(C, rc->bufs);
@@ -1040,6 +1039,8 @@ void ensure_ctx(Scene &sc, int capacity, int trace_grid) {
     P.sort_blk = sc.alloc<int>(nblk * kNumBuckets, rc->bufs);
     P.ctr = sc.alloc<int>(C_ALLOC, rc->bufs);
     P.stat = sc.alloc<unsigned long long>(S_NUM, rc->bufs);
+    P.waves = rc->trace_grid * 4;
+    P.wave_stat = sc.alloc<unsigned long long>(size_t(P.waves), rc->bufs);
     P.spill = sc.alloc<int>(size_t(rc->trace_grid) * 256 * sc.spill_entries, rc->bufs);
     P.accum = sc.alloc<double>(size_t(sc.width) * sc.height * 3, rc->bufs);
     vol_alloc(sc.has_media, C, P, rc->bufs, [&](size_t bytes) {
@@ -1058,8 +1059,7 @@ void launch(K kernel, int grid, int block, hipStream_t s, A... args) {
     HIPX(hipGetLastError());
 }
 
-// The shading kernels of one bounce work on disjoint buckets (their only
-// shared writes are atomic appends to the shadow queue), so with fan set
+// The shading kernels of one bounce work on disjoint buckets, so with fan set
 // they run on three streams at once: a long kernel at one wave per SIMD
 // (DisneyBSDF) leaves most of each SIMD to the others, and the launches'
 // tails overlap.  Captured work (batches) keeps them on one stream.
@@ -1321,8 +1321,7 @@ void render_impl(Scene &sc, const ljx_render_options *o, const ljx_exec_options 
     tm.begin(3, ev);
     launch(k_fill_f64, 1024, 256, s, P.accum, size_t(W) * H * 3);
     launch(k_reset_counters, 1, 64, s, P.ctr, 0, C_ALLOC);
-    hipLaunchKernelGGL(k_reset_stats, dim3(1), dim3(64), 0, s, P.stat);
-    HIPX(hipGetLastError());
+    launch(k_reset_stats, 1, 1024, s, P);
     tm.end(3, ev);
 
     uint64_t passes = 0, train_samples = 0, train_steps = 0, train_step_samples = 0;
@@ -1416,6 +1415,7 @@ void render_impl(Scene &sc, const ljx_render_options *o, const ljx_exec_options 
     size_t nout = size_t(W) * H * 3;
     launch(k_resolve, std::max<int>(1, int(std::min<size_t>(nout / 256 + 1, 4096))), 256, s, (const double *)P.accum,
            out_dev, nout, 1.0 / double(spp));
+    launch(k_sum_stats, 1, 1024, s, P);
     tm.end(3, ev);
     unsigned long long st[S_NUM];
     HIPX(hipMemcpyAsync(st, P.stat, sizeof(st), hipMemcpyDeviceToHost, s));

@@ -32,10 +32,6 @@ constexpr bool kVolpathEnabled = true;
 constexpr uint64_t kNeeStreamXor = 0x5bd1e9955bd1e995ULL;
 constexpr int kMaxShadowSegments = 256;
 
-__global__ void k_reset_stats(unsigned long long *stat) {
-    if (threadIdx.x < S_NUM) stat[threadIdx.x] = 0;
-}
-
 // sigma_t = sigma_s + sigma_a at p
 __device__ __forceinline__ D3 sigma_t_at(const MediumRec &m, D3 p) {
     D3 s, a;
@@ -444,7 +440,6 @@ __global__ __launch_bounds__(256) void k_vol_shade(DeviceScene S, PathBufs P, in
         if (pe) P.alive[pid] = 1;
         int j = wave_append(ps, &P.ctr[C_SH]);
         if (j >= 0) {
-            P.shq[j] = pid;
             P.sh_o[j] = so;
             P.sh_d[j] = sd;
             P.sh_c[j] = sc;
