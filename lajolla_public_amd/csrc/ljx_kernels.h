@@ -43,7 +43,8 @@ constexpr int C_TOTAL = 16 + 4;
 constexpr int kFeeds = 8, kFeedLine = 32, kFeedSet = kFeeds * kFeedLine;
 constexpr int C_FEED = 32;
 constexpr int C_FEED_SHADOW = C_FEED + 2 * kFeedSet;
-constexpr int C_ALLOC = C_FEED + 3 * kFeedSet;
+constexpr int C_FEED_WALK = C_FEED + 3 * kFeedSet;
+constexpr int C_ALLOC = C_FEED + 4 * kFeedSet;
 
 // One job of a batched render: its camera, image and place in the batch's
 // global work index space (sample-major over its 8x8-tiled pixel grid).
@@ -504,6 +505,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? 1 : 8
     if (blockIdx.x == 0 && threadIdx.x < kFeeds) {
         feeds[(cur ^ 1) * kFeedSet + threadIdx.x * kFeedLine] = 0;
         P.ctr[C_FEED_SHADOW + threadIdx.x * kFeedLine] = 0;
+        P.ctr[C_FEED_WALK + threadIdx.x * kFeedLine] = 0;
     }
     const TraceScene ts{S.qnodes, S.prims, S.spheres};
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x;

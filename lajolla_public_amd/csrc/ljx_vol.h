@@ -513,114 +513,186 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? 1 : 8
     }
 }
 
+// One NEE sample's walk towards the light: segments between index-matched
+// boundaries, each with ratio tracking in its medium one collision at a time.
+struct Walk {
+    uint64_t nst, ninc;
+    D3 p0, pp, dir;
+    D3 T, p_nee, p_dir;
+    D3 maj;
+    double max_maj, next_t, accum_t;
+    const MediumRec *m;
+    int pid, bounces, medium, seg, shadow_bounces;
+    int ch, it;
+    int next_medium;   // medium beyond the boundary at the segment's end
+    bool grey, crossings, hit, surface, blocked;
+};
+// Starts a segment: the boundary it ends at (only samples that cross
+// boundaries have one) and its medium's majorant and channel.
+template <bool STATS, bool SPH>
+__device__ __forceinline__ void walk_segment(Walk &w, const DeviceScene &S, int *stack, int *spill, int stride,
+                                             uint32_t &nn, uint32_t &np) {
+    const double dl = sqrt(dist2(w.p0, w.pp));
+    TraceHit h;
+    w.hit = w.crossings && trace_ray<false, STATS, SPH>(TraceScene{S.qnodes, S.prims, S.spheres}, float(w.p0.x),
+                                                        float(w.p0.y), float(w.p0.z), float(w.dir.x), float(w.dir.y),
+                                                        float(w.dir.z), float(S.eps), float((1 - S.eps) * dl), stack,
+                                                        blockDim.x, spill, stride, h, nn, np);
+    w.next_t = dl;
+    if (w.hit) {
+        const Vertex v = make_vertex<SPH>(S, h.slot, h.t, h.u, h.v, w.p0, w.dir);
+        w.next_t = sqrt(dist2(w.p0, v.pos));
+        w.surface = v.material_id >= 0;
+        w.next_medium = update_medium(w.dir, v, w.medium);
+    }
+    if (w.medium >= 0) {
+        w.m = &S.media[w.medium];
+        w.maj = medium_majorant(*w.m, w.p0, w.dir, (1 - S.eps) * dl);
+        w.max_maj = maxc(w.maj);
+        w.grey = w.maj.x == w.maj.y && w.maj.y == w.maj.z;
+        const double u = pcg_double(w.nst, w.ninc);
+        w.ch = min(max(int(u * 3), 0), 2);
+        w.accum_t = 0;
+        w.it = 0;
+    }
+}
+// One collision of the segment's ratio tracking; true at the segment's end.
+__device__ __forceinline__ bool walk_collision(Walk &w, const PathBufs &P) {
+    if (w.medium < 0) return true;
+    const D3 maj = w.maj;
+    const double mc = comp(maj, w.ch);
+    if (mc <= 0) return true;
+    if (w.it >= P.max_null) return true;
+    const double t = -log(1 - pcg_double(w.nst, w.ninc)) / mc;
+    const double dt = w.next_t - w.accum_t;
+    w.accum_t = fmin(w.accum_t + t, w.next_t);
+    if (t < dt) {
+        const D3 sig_t = sigma_t_at(*w.m, w.p0 + w.accum_t * w.dir);
+        const D3 sig_n = maj - sig_t;
+        const D3 e = maj_exp(maj, w.grey, t);
+        w.T = w.T * e * sig_n / w.max_maj;
+        w.p_nee = w.p_nee * e * maj / w.max_maj;
+        const D3 real_prob = sig_t / maj;
+        w.p_dir = w.p_dir * e * maj * (1.0 - real_prob) / w.max_maj;
+        w.it++;
+        return maxc(w.T) <= 0;
+    }
+    const D3 e = maj_exp(maj, w.grey, dt);
+    w.T = w.T * e;
+    w.p_nee = w.p_nee * e;
+    w.p_dir = w.p_dir * e;
+    return true;
+}
+// After a segment: true when the walk has ended.
+__device__ __forceinline__ bool walk_advance(Walk &w, const PathBufs &P) {
+    if (!w.hit) return true;
+    if (w.surface) {
+        w.blocked = true;
+        return true;
+    }
+    w.shadow_bounces++;
+    if (P.max_depth != -1 && w.bounces + w.shadow_bounces + 1 >= P.max_depth) {
+        w.blocked = true;
+        return true;
+    }
+    w.medium = w.next_medium;
+    w.p0 = w.p0 + w.next_t * w.dir;
+    if (++w.seg == kMaxShadowSegments) {
+        w.blocked = true;
+        return true;
+    }
+    return false;
+}
+
 // The NEE shadow walk with ratio tracking (homework2.tex:770-812), after
 // k_vol_occlude: blocked segments are skipped, and only segments that cross
-// index-matched boundaries take closest hits.
+// boundaries take closest hits.  The walks' lengths vary widely (none to
+// hundreds of collisions in a dense grid), so a wave advances all its walks
+// by one collision at a time, and lanes whose walk ended take their next
+// sample once kWalkRefill of them are idle; likewise a segment's start (its
+// closest hit) waits for company.  One lane per sample from start to end
+// left most of a wave idle behind its longest walk: 150 -> 100 ms for the
+// 768x576 64-sample smoke render.
+constexpr int kWalkRefill = 16;
 template <bool STATS, bool SPH>
 __global__ __launch_bounds__(256) void k_vol_shadow(DeviceScene S, PathBufs P) {
     __shared__ int stack[kStackLds * 256];
-    int n = P.ctr[C_SH];
-    int gtid = blockIdx.x * blockDim.x + threadIdx.x;
-    int stride = gridDim.x * blockDim.x;
+    const int n = P.ctr[C_SH];
+    const int gtid = blockIdx.x * blockDim.x + threadIdx.x;
+    const int stride = gridDim.x * blockDim.x;
     int *spill = P.spill + gtid;
     uint32_t nn = 0, np = 0;
-    unsigned long long segs = 0;
-    for (int i = gtid; i < n; i += stride) {
-        float4 so = P.sh_o[i], sd = P.sh_d[i], sc = P.sh_c[i], sx = P.sh_x[i];
-        int pid = __float_as_int(sc.w);
-        int medium = __float_as_int(so.w);
-        int bounces = __float_as_int(sd.w);
-        D3 p{so.x, so.y, so.z}, pp{sd.x, sd.y, sd.z};
-        uint64_t nst = uint64_t(__float_as_uint(sx.z)) | (uint64_t(__float_as_uint(sx.w)) << 32);
-        const uint64_t nstream = slot_info(P, pid).stream() ^ kNeeStreamXor;
-        uint64_t ninc = pcg_inc(nstream);
-        D3 dir_light = normalize(pp - p);
-        D3 T{1, 1, 1}, p_nee{1, 1, 1}, p_dir{1, 1, 1};
-        D3 p0 = p;
-        bool blocked = false;
-        int shadow_bounces = 0;
-        // k_vol_occlude's verdict (the NEE stream is not written back, so
-        // skipping a blocked segment's walk leaves every other draw unchanged)
-        bool crossings = false;
-        if (S.num_nodes > 0) {
-            const uint8_t occ = P.sh_occ[i];
-            if (occ == 1) continue;
-            crossings = occ == 2;
-        }
-        for (int seg = 0; seg < kMaxShadowSegments; seg++) {
-            double dl = sqrt(dist2(p0, pp));
-            TraceHit h;
-            if (crossings) segs++;
-            bool hit = crossings &&
-                       trace_ray<false, STATS, SPH>(TraceScene{S.qnodes, S.prims, S.spheres}, float(p0.x), float(p0.y),
-                                                    float(p0.z), float(dir_light.x), float(dir_light.y),
-                                                    float(dir_light.z), float(S.eps), float((1 - S.eps) * dl),
-                                                    stack + threadIdx.x, blockDim.x, spill, stride, h, nn, np);
-            Vertex v;
-            double next_t = dl;
-            if (hit) {
-                v = make_vertex<SPH>(S, h.slot, h.t, h.u, h.v, p0, dir_light);
-                next_t = sqrt(dist2(p0, v.pos));
-            }
-            if (medium >= 0) {
-                const MediumRec &m = S.media[medium];
-                D3 maj = medium_majorant(m, p0, dir_light, (1 - S.eps) * dl);
-                double max_maj = maxc(maj);
-                const bool grey = maj.x == maj.y && maj.y == maj.z;
-                double u = pcg_double(nst, ninc);
-                int ch = min(max(int(u * 3), 0), 2);
-                double accum_t = 0;
-                for (int it = 0;; it++) {
-                    double mc = comp(maj, ch);
-                    if (mc <= 0) break;
-                    if (it >= P.max_null) break;
-                    double t = -log(1 - pcg_double(nst, ninc)) / mc;
-                    double dt = next_t - accum_t;
-                    accum_t = fmin(accum_t + t, next_t);
-                    if (t < dt) {
-                        D3 sig_t = sigma_t_at(m, p0 + accum_t * dir_light);
-                        D3 sig_n = maj - sig_t;
-                        D3 e = maj_exp(maj, grey, t);
-                        T = T * e * sig_n / max_maj;
-                        p_nee = p_nee * e * maj / max_maj;
-                        D3 real_prob = sig_t / maj;
-                        p_dir = p_dir * e * maj * (1.0 - real_prob) / max_maj;
-                        if (maxc(T) <= 0) break;
-                    } else {
-                        D3 e = maj_exp(maj, grey, dt);
-                        T = T * e;
-                        p_nee = p_nee * e;
-                        p_dir = p_dir * e;
-                        break;
-                    }
+    int segs = 0;
+    Walk w;
+    int i = 0;
+    // a busy lane is at a segment's start (wait) or inside one
+    bool busy = false, fin = false, wait = false;
+    FeedRange range;
+    range.start(P.ctr + C_FEED_WALK, n);
+    while (true) {
+        const uint64_t idle = __ballot(!busy);
+        const int nidle = __popcll(idle);
+        if (nidle >= kWalkRefill) {
+            if (fin && !w.blocked && maxc(w.T) > 0) {
+                const float4 sc = P.sh_c[i], sx = P.sh_x[i];
+                const double pdf_nee = double(sx.x) * avgc(w.p_nee);
+                if (pdf_nee > 0) {
+                    const double pdf_dir = double(sx.y) * avgc(w.p_dir);
+                    const double wt = (pdf_nee * pdf_nee) / (pdf_nee * pdf_nee + pdf_dir * pdf_dir);
+                    const D3 c = D3{sc.x, sc.y, sc.z} * w.T * (wt / pdf_nee);
+                    const float4 r = P.rad[w.pid];
+                    P.rad[w.pid] = make_float4(float(r.x + c.x), float(r.y + c.y), float(r.z + c.z), 0.f);
                 }
             }
-            if (!hit) break;
-            if (v.material_id >= 0) {
-                blocked = true;
-                break;
+            fin = false;
+            range.refill();
+            const int k = range.take(int(__builtin_amdgcn_mbcnt_hi(uint32_t(idle >> 32),
+                                                                   __builtin_amdgcn_mbcnt_lo(uint32_t(idle), 0))),
+                                     nidle);
+            if (!busy && k >= 0) {
+                // k_vol_occlude's verdict (the NEE stream is not written back,
+                // so skipping a blocked sample leaves every other draw
+                // unchanged)
+                const uint8_t occ = S.num_nodes > 0 ? P.sh_occ[k] : uint8_t(0);
+                if (occ != 1) {
+                    i = k;
+                    const float4 so = P.sh_o[i], sd = P.sh_d[i], sx = P.sh_x[i];
+                    w.pid = __float_as_int(P.sh_c[i].w);
+                    w.medium = __float_as_int(so.w);
+                    w.bounces = __float_as_int(sd.w);
+                    w.p0 = D3{so.x, so.y, so.z};
+                    w.pp = D3{sd.x, sd.y, sd.z};
+                    w.dir = normalize(w.pp - w.p0);
+                    w.nst = uint64_t(__float_as_uint(sx.z)) | (uint64_t(__float_as_uint(sx.w)) << 32);
+                    w.ninc = pcg_inc(slot_info(P, w.pid).stream() ^ kNeeStreamXor);
+                    w.T = w.p_nee = w.p_dir = D3{1, 1, 1};
+                    w.crossings = occ == 2;
+                    w.seg = w.shadow_bounces = 0;
+                    w.blocked = false;
+                    busy = wait = true;
+                }
             }
-            shadow_bounces++;
-            if (P.max_depth != -1 && bounces + shadow_bounces + 1 >= P.max_depth) {
-                blocked = true;
-                break;
+            if (__ballot(busy) == 0) {
+                if (range.done) break;
+                continue;
             }
-            medium = update_medium(dir_light, v, medium);
-            p0 = p0 + next_t * dir_light;
-            if (seg == kMaxShadowSegments - 1) blocked = true;
         }
-        if (!blocked && maxc(T) > 0) {
-            double pdf_nee = double(sx.x) * avgc(p_nee);
-            if (pdf_nee > 0) {
-                double pdf_dir = double(sx.y) * avgc(p_dir);
-                double w = (pdf_nee * pdf_nee) / (pdf_nee * pdf_nee + pdf_dir * pdf_dir);
-                D3 c = D3{sc.x, sc.y, sc.z} * T * (w / pdf_nee);
-                float4 r = P.rad[pid];
-                P.rad[pid] = make_float4(float(r.x + c.x), float(r.y + c.y), float(r.z + c.z), 0.f);
+        const int nwait = __popcll(__ballot(wait));
+        if (nwait >= kWalkRefill || (nwait > 0 && __ballot(busy && !wait) == 0)) {
+            segs += __popcll(__ballot(wait && w.crossings));
+            if (wait) walk_segment<STATS, SPH>(w, S, stack + threadIdx.x, spill, stride, nn, np);
+            wait = false;
+        }
+        if (busy && !wait && walk_collision(w, P)) {
+            if (walk_advance(w, P)) {
+                busy = false;
+                fin = true;
+            } else {
+                wait = true;
             }
         }
     }
-    atomicAdd(&P.stat[S_SH_RAYS], segs);
+    if (__lane_id() == 0) P.wave_stat[gtid >> 6] += (unsigned long long)segs;
     if (STATS) {
         atomicAdd(&P.stat[S_SH_NODES], (unsigned long long)nn);
         atomicAdd(&P.stat[S_SH_PRIMS], (unsigned long long)np);
