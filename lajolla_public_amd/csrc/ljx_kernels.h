@@ -33,10 +33,8 @@ constexpr int kBucketNoMat = 11;
 constexpr int kNumBuckets = 12;
 // counter slots
 constexpr int C_EXT = 0;      // C_EXT + (0|1): extension queues
-constexpr int C_SH = 2;       // shadow queue (volumetric)
 constexpr int C_BUCKET = 4;   // C_BUCKET + bucket: its paths
-constexpr int C_FLQ = 18;     // volumetric free-flight queue: its length, then (C_FLQ + 1) paths taken from it
-constexpr int C_TOTAL = 16 + 4;
+constexpr int C_TOTAL = 16;
 // ticket counters (Feed), in sets of kFeeds a 128-byte line apart: two for
 // the closest-hit launches, used in turn by the bounces, and one each for the
 // bounce's other launches
@@ -44,7 +42,8 @@ constexpr int kFeeds = 8, kFeedLine = 32, kFeedSet = kFeeds * kFeedLine;
 constexpr int C_FEED = 32;
 constexpr int C_FEED_SHADOW = C_FEED + 2 * kFeedSet;
 constexpr int C_FEED_WALK = C_FEED + 3 * kFeedSet;
-constexpr int C_ALLOC = C_FEED + 4 * kFeedSet;
+constexpr int C_FEED_FLIGHT = C_FEED + 4 * kFeedSet;
+constexpr int C_ALLOC = C_FEED + 5 * kFeedSet;
 
 // One job of a batched render: its camera, image and place in the batch's
 // global work index space (sample-major over its 8x8-tiled pixel grid).
@@ -88,7 +87,6 @@ struct PathBufs {
     float4 *sh_x;     // shadow walk: pdf_nee, pdf_dir, NEE stream state (lo, hi bits)
     double4 *vf_t;    // free flight: transmittance rgb, distance travelled
     double4 *vf_p;    // free flight: transmittance pdf rgb, 1 if it ended in a real collision
-    uint32_t *flq;    // free flight: the paths of the volumetric queue that are in a medium
     int *ctr;
     unsigned long long *stat;
     int *spill;
@@ -126,8 +124,8 @@ struct PathBufs {
     long long valid0;
 };
 
-// A surface vertex's shadow ray is written at its path's place in P.order;
-// places without one carry this mark in sh_occ.
+// A vertex's shadow ray is written at its path's place in P.order (volumetric:
+// in the extension queue); places without one carry this mark in sh_occ.
 constexpr uint8_t kShNone = 3;
 // Shadow-queue entries carry the path slot in the low kSlotBits bits and the
 // vertex index in the rest (clamped there: only the guiding record, a few
@@ -428,29 +426,40 @@ __global__ void k_raygen(DeviceScene S, PathBufs P) {
 // kFeedRun chunks: an XCD's waves work on neighbouring entries, and every feed
 // sees all parts of the queue.
 constexpr int kFeedRun = 16;
+// A ticket's round trip takes over a microsecond, which two or three waves per
+// SIMD do not hide.  For kernels of such occupancy a ticket covers several
+// chunks of a long queue, as many as leave every wave `tickets` of them (media
+// render's shadow walks 14.9 -> 7.5 ms); at eight waves per SIMD single chunks
+// are better (terrain's closest hits 56.4 against 58.8 ms).
+constexpr int kFeedTickets = 8;
 struct Feed {
-    int feeds, feed, waves, ticket;
+    int feeds, feed, waves, ticket, sub, span;
     int *counter;
-    bool more;  // chunks remain after every wave's first
+    bool more;  // tickets remain after every wave's first
     __device__ __forceinline__ int chunk(int t) const {
-        return ((t / kFeedRun) * feeds + feed) * kFeedRun + t % kFeedRun;
+        return ((t * span / kFeedRun) * feeds + feed) * kFeedRun + t * span % kFeedRun;
     }
     // counters: a set of kFeeds zeroed counters kFeedLine apart.  Grids of
     // fewer than kFeeds blocks use one feed.
-    __device__ __forceinline__ void start(int *counters, int n) {
-        const int wpb = blockDim.x >> 6;
+    __device__ __forceinline__ void start(int *counters, int n, int tickets = 0) {
+        const int wpb = blockDim.x >> 6, chunks = (n + 63) / 64;
         feeds = int(gridDim.x) < kFeeds ? 1 : kFeeds;
         feed = int(blockIdx.x) % feeds;
         waves = (int(gridDim.x) + feeds - 1 - feed) / feeds * wpb;
+        span = 1;
+        while (tickets > 0 && span < kFeedRun && chunks >= 2 * span * tickets * int(gridDim.x) * wpb) span *= 2;
         ticket = __builtin_amdgcn_readfirstlane(int(blockIdx.x) / feeds * wpb + int(threadIdx.x >> 6));
+        sub = 0;
         counter = counters + feed * kFeedLine;
-        more = chunk(waves) < (n + 63) / 64;
+        more = chunk(waves) < chunks;
     }
     // First entry of the wave's current chunk; at or past n: none is left.
-    __device__ __forceinline__ int base() const { return chunk(ticket) * 64; }
+    __device__ __forceinline__ int base() const { return (chunk(ticket) + sub) * 64; }
     __device__ __forceinline__ void next(int n) {
+        if (++sub < span) return;
+        sub = 0;
         if (!more) {
-            ticket = 1 << 20;  // past every queue (2^26 entries)
+            ticket = (1 << 20) / span;  // past every queue (2^26 entries)
             return;
         }
         int t = 0;
@@ -498,7 +507,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? 1 : 8
     const int n = P.ctr[C_EXT + cur];
     const bool sorted = n >= P.sort_threshold;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        P.ctr[C_SH] = 0;
         atomicAdd(&P.stat[S_EXT_RAYS], (unsigned long long)n);
     }
     int *feeds = P.ctr + C_FEED;
@@ -506,6 +514,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? 1 : 8
         feeds[(cur ^ 1) * kFeedSet + threadIdx.x * kFeedLine] = 0;
         P.ctr[C_FEED_SHADOW + threadIdx.x * kFeedLine] = 0;
         P.ctr[C_FEED_WALK + threadIdx.x * kFeedLine] = 0;
+        P.ctr[C_FEED_FLIGHT + threadIdx.x * kFeedLine] = 0;
     }
     const TraceScene ts{S.qnodes, S.prims, S.spheres};
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x;
@@ -794,35 +803,54 @@ __global__ __launch_bounds__(256) void k_miss(DeviceScene S, PathBufs P) {
     }
 }
 
-// A wave's current range of a queue it takes lane by lane (k_shadow): chunks
-// of 64 entries from a Feed.
+// Hands a wave's lanes the entries of a queue one by one, passing over those
+// that need no work: chunks of 64 entries from a Feed, the entries of a chunk
+// to work on gathered in `list` (lane k holds the k-th of them).
 struct FeedRange {
     Feed feed;
-    int cursor, end, n;
-    bool done;  // the feed has no more chunks
-    __device__ __forceinline__ void open() {
-        cursor = feed.base();
-        done = cursor >= n;
-        if (done) cursor = n;
-        end = min(n, cursor + 64);
-    }
-    __device__ __forceinline__ void start(int *counters, int n_) {
+    int n, list, at, count;
+    bool fresh;  // the feed's current chunk has not been opened
+    bool done;   // no entries are left
+    __device__ __forceinline__ void start(int *counters, int n_, int tickets = 0) {
         n = n_;
-        feed.start(counters, n);
-        open();
+        feed.start(counters, n, tickets);
+        at = count = 0;
+        fresh = true;
+        done = false;
     }
-    // A new chunk once the current one is used up.
-    __device__ __forceinline__ void refill() {
-        if (cursor < end || done) return;
-        feed.next(n);
-        open();
-    }
-    // The entry of the k-th of the wave's asking lanes (asked of them in
-    // total), or -1.
-    __device__ __forceinline__ int take(int k, int asked) {
-        const int i = cursor + k < end ? cursor + k : -1;
-        cursor = min(end, cursor + asked);
-        return i;
+    // One entry with valid(entry) for every lane that wants one, or -1 once
+    // none are left.  All lanes of the wave must call it.
+    template <class F>
+    __device__ __forceinline__ int take(bool want, F &&valid) {
+        int got = -1;
+        uint64_t w = __ballot(want);
+        auto below = [](uint64_t m) {
+            return int(__builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), 0)));
+        };
+        while (w && !done) {
+            if (at == count) {
+                if (!fresh) feed.next(n);
+                fresh = false;
+                const int base = feed.base();
+                if (base >= n) {
+                    done = true;
+                    break;
+                }
+                const int lane = __lane_id(), i = base + lane;
+                const bool v = i < n && valid(i);
+                const uint64_t m = __ballot(v);
+                const int r = below(m);
+                at = 0;
+                count = __popcll(m);
+                list = __builtin_amdgcn_ds_permute(4 * (v ? r : count + lane - r), i);
+            }
+            const int k = at + below(w);
+            const int e = __shfl(list, k < 63 ? k : 63);
+            if (want && got < 0 && k < count) got = e;
+            at = min(count, at + __popcll(w));
+            w = __ballot(want && got < 0);
+        }
+        return got;
     }
 };
 
@@ -831,8 +859,7 @@ struct FeedRange {
 // contributions).  A lane whose ray ended takes its next one as soon as
 // kShadowRefill lanes of its wave are idle, instead of waiting for the
 // wave's longest ray (3.6% faster on the 1080p large-mesh render than
-// starting the lanes' rays together); places without a ray leave their lane
-// idle until the next such turn.
+// starting the lanes' rays together).
 constexpr int kShadowRefill = 16;
 template <bool STATS, bool SPH>
 __global__ __launch_bounds__(256) void k_shadow(DeviceScene S, PathBufs P) {
@@ -851,14 +878,11 @@ __global__ __launch_bounds__(256) void k_shadow(DeviceScene S, PathBufs P) {
     while (true) {
         const uint64_t idle = __ballot(!busy);
         const int nidle = __popcll(idle);
-        if (nidle >= kShadowRefill) {
+        if ((nidle >= kShadowRefill && !range.done) || nidle == 64) {
             if (fin) P.sh_occ[i] = tr.found ? 1 : 0;
             fin = false;
-            range.refill();
-            const int k = range.take(int(__builtin_amdgcn_mbcnt_hi(uint32_t(idle >> 32),
-                                                                   __builtin_amdgcn_mbcnt_lo(uint32_t(idle), 0))),
-                                     nidle);
-            if (!busy && k >= 0 && P.sh_occ[k] != kShNone) {
+            const int k = range.take(!busy, [&](int j) { return P.sh_occ[j] != kShNone; });
+            if (k >= 0) {
                 i = k;
                 const float4 o = P.sh_o[i], d = P.sh_d[i];
                 tr.start(o.x, o.y, o.z, d.x, d.y, d.z, o.w, d.w);
@@ -866,10 +890,7 @@ __global__ __launch_bounds__(256) void k_shadow(DeviceScene S, PathBufs P) {
             }
             const int now = __popcll(__ballot(busy));
             rays += now - (64 - nidle);
-            if (now == 0) {
-                if (range.done) break;
-                continue;
-            }
+            if (now == 0) break;
         }
         if (busy) {
             if (S.num_nodes == 0 || tr.step(ts, stack + threadIdx.x, blockDim.x, spill, stride, nn, np)) {

@@ -1379,7 +1379,7 @@ void render_impl(Scene &sc, const ljx_render_options *o, const ljx_exec_options 
                 build_ext_queue(P, ns * nq, cur, s);
                 tm.end(2, ev);
                 tm.begin(1, ev);
-                if (vol) vol_shadow(S, P, tgrid, s, stats_on, sc.has_spheres);
+                if (vol) vol_shadow(S, P, cur, tgrid, s, stats_on, sc.has_spheres);
                 else trace_stage(sc, P, cur, tgrid, shade_grid, s, stats_on, true);
                 tm.end(1, ev);
                 cur ^= 1;
@@ -1697,7 +1697,7 @@ void batch_impl(const ljx_batch_job *jobs, size_t njobs, const ljx_exec_options 
                     if (vol) vol_shade_all(S, P, cur, sgrid, cs, sc.has_spheres, (sc.mat_types_present & ~7u) == 0);
                     else shade_all(sc, P, cur, sgrid, cs, false, gp.block);
                     build_ext_queue(P, n, cur, cs);
-                    if (vol) vol_shadow(S, P, tgrid, cs, false, sc.has_spheres);
+                    if (vol) vol_shadow(S, P, cur, tgrid, cs, false, sc.has_spheres);
                     else trace_stage(sc, P, cur, tgrid, sgrid, cs, false, true);
                     cur ^= 1;
                 }

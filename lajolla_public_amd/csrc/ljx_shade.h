@@ -1,27 +1,10 @@
-// Hit reconstruction, light sampling and wave-level queue helpers shared by
-// the wavefront kernels.
+// Hit reconstruction and light sampling shared by the wavefront kernels.
 #pragma once
 
 #include "ljx_device.h"
 #include "ljx_trace.h"
 
 namespace ljx {
-
-// ------------------------------------------------------------ wave helpers
-// Appends the lanes with pred set to a queue guarded by *counter: one atomic
-// per wave (ballot + popcount), lane offsets from mbcnt.  Every lane of the
-// wave must call it.  Returns the lane's queue index, or -1.
-__device__ __forceinline__ int wave_append(bool pred, int *counter) {
-    uint64_t mask = __ballot(pred);
-    if (mask == 0) return -1;
-    int lane = __lane_id();
-    int leader = __ffsll((unsigned long long)mask) - 1;
-    int base = 0;
-    if (lane == leader) base = atomicAdd(counter, __popcll(mask));
-    base = __shfl(base, leader);
-    int below = __builtin_amdgcn_mbcnt_hi(uint32_t(mask >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(mask), 0));
-    return pred ? base + below : -1;
-}
 
 __device__ __forceinline__ D3 f3d(float4 v) { return D3{double(v.x), double(v.y), double(v.z)}; }
 

@@ -148,62 +148,25 @@ __device__ __forceinline__ double hit_distance(const DeviceScene &S, float4 h, D
     return sqrt(dist2(org, v.pos));
 }
 
-// The paths of the volumetric queue that are in a medium, for k_vol_flight
-// (the order does not matter: each path's flight uses its own stream).  Each
-// block of 1,024 threads appends with one atomic per round (a wave per
-// atomic contended on the one counter).
-__global__ __launch_bounds__(1024) void k_vol_flight_queue(PathBufs P, int cur) {
-    __shared__ int wcount[16];
-    __shared__ int bbase;
-    const int n = P.ctr[C_EXT + cur];
-    const uint32_t *q = cur ? P.extq1 : P.extq0;
-    const int stride = gridDim.x * blockDim.x;
-    const int w = threadIdx.x >> 6;
-    for (int base = blockIdx.x * blockDim.x; base < n; base += stride) {
-        const int i = base + threadIdx.x;
-        uint32_t pid = 0;
-        bool in_medium = false;
-        if (i < n) {
-            pid = q[i];
-            in_medium = P.medium[pid] >= 0;
-        }
-        const uint64_t mask = __ballot(in_medium);
-        if ((threadIdx.x & 63) == 0) wcount[w] = __popcll(mask);
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            int total = 0;
-            for (int k = 0; k < 16; k++) total += wcount[k];
-            bbase = total > 0 ? atomicAdd(&P.ctr[C_FLQ], total) : 0;
-        }
-        __syncthreads();
-        if (in_medium) {
-            int k = bbase + int(__builtin_amdgcn_mbcnt_hi(uint32_t(mask >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(mask), 0)));
-            for (int q = 0; q < w; q++) k += wcount[q];
-            P.flq[k] = pid;
-        }
-        __syncthreads();
-    }
-}
-
-// Free flight for every path of the flight queue, in a kernel small enough
-// for three waves per SIMD.  The loops' lengths vary widely between paths, so
-// a lane whose flight ended takes its next path as soon as kFlightRefill
-// lanes of its wave are idle (one atomic per wave for all of them) rather
+// Free flight for the queue's paths that are in a medium, in a kernel small
+// enough for three waves per SIMD.  The loops' lengths vary widely between
+// paths, so a lane whose flight ended (or whose path is in no medium) takes
+// its next path as soon as kFlightRefill lanes of its wave are idle rather
 // than waiting for the wave's longest flight.
 constexpr int kFlightRefill = 16;
 template <bool SPH>
-__global__ __launch_bounds__(256) void k_vol_flight(DeviceScene S, PathBufs P) {
-    const int n = P.ctr[C_FLQ];
-    int *fetch = &P.ctr[C_FLQ + 1];
-    const int lane = __lane_id();
+__global__ __launch_bounds__(256) void k_vol_flight(DeviceScene S, PathBufs P, int cur) {
+    const uint32_t *q = cur ? P.extq1 : P.extq0;
     FlightRun r;
     uint64_t st = 0, inc = 0;
     uint32_t pid = 0;
-    bool busy = false, fin = false, more = true;  // more: wave-uniform
+    bool busy = false, fin = false;
+    FeedRange range;
+    range.start(P.ctr + C_FEED_FLIGHT, P.ctr[C_EXT + cur], kFeedTickets);
     while (true) {
         const uint64_t idle = __ballot(!busy);
         const int nidle = __popcll(idle);
-        if ((more && nidle >= kFlightRefill) || nidle == 64) {
+        if ((nidle >= kFlightRefill && !range.done) || nidle == 64) {
             if (fin) {
                 P.rng[pid] = st;
                 P.vf_t[pid] = make_double4(r.fl.T.x, r.fl.T.y, r.fl.T.z, r.fl.accum_t);
@@ -211,15 +174,9 @@ __global__ __launch_bounds__(256) void k_vol_flight(DeviceScene S, PathBufs P) {
                                            r.fl.scatter ? 1.0 : 0.0);
                 fin = false;
             }
-            if (!more) break;  // every lane idle and the queue drained
-            int base = 0;
-            if (lane == 0) base = atomicAdd(fetch, nidle);
-            base = __shfl(base, 0);
-            if (base + nidle >= n) more = false;
-            const int i = base + int(__builtin_amdgcn_mbcnt_hi(uint32_t(idle >> 32),
-                                                               __builtin_amdgcn_mbcnt_lo(uint32_t(idle), 0)));
-            if (!busy && i < n) {
-                pid = P.flq[i];
+            const int i = range.take(!busy, [&](int j) { return P.medium[q[j]] >= 0; });
+            if (i >= 0) {
+                pid = q[i];
                 const float4 ro = P.ray_o[pid], rd = P.ray_d[pid];
                 const D3 org = f3d(ro), dir = f3d(rd);
                 st = P.rng[pid];
@@ -227,6 +184,7 @@ __global__ __launch_bounds__(256) void k_vol_flight(DeviceScene S, PathBufs P) {
                 flight_begin(r, S, P.medium[pid], org, dir, hit_distance<SPH>(S, P.hit[pid], org, dir), st, inc);
                 busy = true;
             }
+            if (__ballot(busy) == 0) break;
         }
         if (busy && flight_step(r, P, st, inc)) {
             busy = false;
@@ -428,22 +386,20 @@ __global__ __launch_bounds__(256) void k_vol_shade(DeviceScene S, PathBufs P, in
     int n = P.ctr[C_EXT + cur];
     const uint32_t *q = cur ? P.extq1 : P.extq0;
     int stride = gridDim.x * blockDim.x;
-    for (int base = blockIdx.x * blockDim.x; base < n; base += stride) {
-        int i = base + threadIdx.x;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+        const uint32_t pid = q[i];
         bool pe = false, ps = false;
         float4 so, sd, sc, sx;
-        uint32_t pid = 0;
-        if (i < n) {
-            pid = q[i];
-            vol_shade<SPH, DMT>(S, P, pid, pe, ps, so, sd, sc, sx);
-        }
+        vol_shade<SPH, DMT>(S, P, pid, pe, ps, so, sd, sc, sx);
         if (pe) P.alive[pid] = 1;
-        int j = wave_append(ps, &P.ctr[C_SH]);
-        if (j >= 0) {
-            P.sh_o[j] = so;
-            P.sh_d[j] = sd;
-            P.sh_c[j] = sc;
-            P.sh_x[j] = sx;
+        // the shadow ray takes its path's place in the queue (shade_queue):
+        // appending it took one of 11.3 ns after the other per wave
+        P.sh_occ[i] = ps ? uint8_t(0) : kShNone;
+        if (ps) {
+            P.sh_o[i] = so;
+            P.sh_d[i] = sd;
+            P.sh_c[i] = sc;
+            P.sh_x[i] = sx;
         }
     }
 }
@@ -460,33 +416,26 @@ __global__ __launch_bounds__(256) void k_vol_shade(DeviceScene S, PathBufs P, in
 // waves per SIMD.  Triangle-only scenes cap it at eight waves per SIMD (64
 // registers, a 16-byte spill).
 template <bool STATS, bool SPH>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? 1 : 8))) void k_vol_occlude(DeviceScene S, PathBufs P) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? 1 : 8))) void k_vol_occlude(DeviceScene S, PathBufs P, int cur) {
     __shared__ int stack[kStackLds * 256];
-    const int n = P.ctr[C_SH];
     const TraceScene ts{S.qnodes, S.prims, S.spheres, S.slot_passthru};
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x;
     const int stride = gridDim.x * blockDim.x;
     int *spill = P.spill + gtid;
     uint32_t nn = 0, np = 0;
-    unsigned long long segs = 0;
     Tracer<true, STATS, SPH, true> tr;
     bool busy = false, fin = false;
-    // each wave walks its own contiguous share of the queue (k_shadow)
-    const int nwaves = stride >> 6;
-    const int per = (n + nwaves - 1) / nwaves;
-    int cursor = (gtid >> 6) * per;
-    const int end = min(n, cursor + per);
-    int i = 0;
+    FeedRange range;
+    range.start(P.ctr + C_FEED_SHADOW, P.ctr[C_EXT + cur]);
+    int i = 0, rays = 0;
     while (true) {
         const uint64_t idle = __ballot(!busy);
         const int nidle = __popcll(idle);
-        if (nidle >= kShadowRefill) {
+        if ((nidle >= kShadowRefill && !range.done) || nidle == 64) {
             if (fin) P.sh_occ[i] = tr.found ? 1 : (tr.passed ? 2 : 0);
             fin = false;
-            const int k = cursor + int(__builtin_amdgcn_mbcnt_hi(uint32_t(idle >> 32),
-                                                                 __builtin_amdgcn_mbcnt_lo(uint32_t(idle), 0)));
-            cursor = min(end, cursor + nidle);
-            if (!busy && k < end) {
+            const int k = range.take(!busy, [&](int j) { return P.sh_occ[j] != kShNone; });
+            if (k >= 0) {
                 i = k;
                 const float4 so = P.sh_o[i], sd = P.sh_d[i];
                 const D3 p{so.x, so.y, so.z}, pp{sd.x, sd.y, sd.z};
@@ -495,9 +444,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? 1 : 8
                 tr.start(float(p.x), float(p.y), float(p.z), float(dir_light.x), float(dir_light.y),
                          float(dir_light.z), float(S.eps), float((1 - S.eps) * dl));
                 busy = true;
-                if (S.num_nodes > 0) segs++;
             }
-            if (__ballot(busy) == 0) break;
+            const int now = __popcll(__ballot(busy));
+            rays += now - (64 - nidle);
+            if (now == 0) break;
         }
         if (busy) {
             if (S.num_nodes == 0 || tr.step(ts, stack + threadIdx.x, blockDim.x, spill, stride, nn, np)) {
@@ -506,7 +456,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? 1 : 8
             }
         }
     }
-    atomicAdd(&P.stat[S_SH_RAYS], segs);
+    if (S.num_nodes > 0 && __lane_id() == 0) P.wave_stat[gtid >> 6] += (unsigned long long)rays;
     if (STATS) {
         atomicAdd(&P.stat[S_SH_NODES], (unsigned long long)nn);
         atomicAdd(&P.stat[S_SH_PRIMS], (unsigned long long)np);
@@ -615,9 +565,8 @@ __device__ __forceinline__ bool walk_advance(Walk &w, const PathBufs &P) {
 // 768x576 64-sample smoke render.
 constexpr int kWalkRefill = 16;
 template <bool STATS, bool SPH>
-__global__ __launch_bounds__(256) void k_vol_shadow(DeviceScene S, PathBufs P) {
+__global__ __launch_bounds__(256) void k_vol_shadow(DeviceScene S, PathBufs P, int cur) {
     __shared__ int stack[kStackLds * 256];
-    const int n = P.ctr[C_SH];
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x;
     const int stride = gridDim.x * blockDim.x;
     int *spill = P.spill + gtid;
@@ -628,11 +577,11 @@ __global__ __launch_bounds__(256) void k_vol_shadow(DeviceScene S, PathBufs P) {
     // a busy lane is at a segment's start (wait) or inside one
     bool busy = false, fin = false, wait = false;
     FeedRange range;
-    range.start(P.ctr + C_FEED_WALK, n);
+    range.start(P.ctr + C_FEED_WALK, P.ctr[C_EXT + cur], kFeedTickets);
     while (true) {
         const uint64_t idle = __ballot(!busy);
         const int nidle = __popcll(idle);
-        if (nidle >= kWalkRefill) {
+        if ((nidle >= kWalkRefill && !range.done) || nidle == 64) {
             if (fin && !w.blocked && maxc(w.T) > 0) {
                 const float4 sc = P.sh_c[i], sx = P.sh_x[i];
                 const double pdf_nee = double(sx.x) * avgc(w.p_nee);
@@ -645,37 +594,31 @@ __global__ __launch_bounds__(256) void k_vol_shadow(DeviceScene S, PathBufs P) {
                 }
             }
             fin = false;
-            range.refill();
-            const int k = range.take(int(__builtin_amdgcn_mbcnt_hi(uint32_t(idle >> 32),
-                                                                   __builtin_amdgcn_mbcnt_lo(uint32_t(idle), 0))),
-                                     nidle);
-            if (!busy && k >= 0) {
-                // k_vol_occlude's verdict (the NEE stream is not written back,
-                // so skipping a blocked sample leaves every other draw
-                // unchanged)
-                const uint8_t occ = S.num_nodes > 0 ? P.sh_occ[k] : uint8_t(0);
-                if (occ != 1) {
-                    i = k;
-                    const float4 so = P.sh_o[i], sd = P.sh_d[i], sx = P.sh_x[i];
-                    w.pid = __float_as_int(P.sh_c[i].w);
-                    w.medium = __float_as_int(so.w);
-                    w.bounces = __float_as_int(sd.w);
-                    w.p0 = D3{so.x, so.y, so.z};
-                    w.pp = D3{sd.x, sd.y, sd.z};
-                    w.dir = normalize(w.pp - w.p0);
-                    w.nst = uint64_t(__float_as_uint(sx.z)) | (uint64_t(__float_as_uint(sx.w)) << 32);
-                    w.ninc = pcg_inc(slot_info(P, w.pid).stream() ^ kNeeStreamXor);
-                    w.T = w.p_nee = w.p_dir = D3{1, 1, 1};
-                    w.crossings = occ == 2;
-                    w.seg = w.shadow_bounces = 0;
-                    w.blocked = false;
-                    busy = wait = true;
-                }
+            // k_vol_occlude's verdict picks the samples (the NEE stream is not
+            // written back, so skipping a blocked one leaves every other draw
+            // unchanged)
+            const int k = range.take(!busy, [&](int j) {
+                const uint8_t occ = P.sh_occ[j];
+                return occ == 0 || occ == 2;
+            });
+            if (k >= 0) {
+                i = k;
+                const float4 so = P.sh_o[i], sd = P.sh_d[i], sx = P.sh_x[i];
+                w.pid = __float_as_int(P.sh_c[i].w);
+                w.medium = __float_as_int(so.w);
+                w.bounces = __float_as_int(sd.w);
+                w.p0 = D3{so.x, so.y, so.z};
+                w.pp = D3{sd.x, sd.y, sd.z};
+                w.dir = normalize(w.pp - w.p0);
+                w.nst = uint64_t(__float_as_uint(sx.z)) | (uint64_t(__float_as_uint(sx.w)) << 32);
+                w.ninc = pcg_inc(slot_info(P, w.pid).stream() ^ kNeeStreamXor);
+                w.T = w.p_nee = w.p_dir = D3{1, 1, 1};
+                w.crossings = P.sh_occ[i] == 2;
+                w.seg = w.shadow_bounces = 0;
+                w.blocked = false;
+                busy = wait = true;
             }
-            if (__ballot(busy) == 0) {
-                if (range.done) break;
-                continue;
-            }
+            if (__ballot(busy) == 0) break;
         }
         const int nwait = __popcll(__ballot(wait));
         if (nwait >= kWalkRefill || (nwait > 0 && __ballot(busy && !wait) == 0)) {
@@ -724,7 +667,6 @@ void vol_alloc(bool, size_t capacity, PathBufs &P, Bufs &bufs, Alloc alloc) {
     P.sh_x = static_cast<float4 *>(take(capacity * sizeof(float4)));
     P.vf_t = static_cast<double4 *>(take(capacity * sizeof(double4)));
     P.vf_p = static_cast<double4 *>(take(capacity * sizeof(double4)));
-    P.flq = static_cast<uint32_t *>(take(capacity * sizeof(uint32_t)));
 }
 
 inline void vol_launch_check() {
@@ -735,10 +677,8 @@ inline void vol_launch_check() {
 // basic: the scene uses no material types beyond lajolla's three basic ones.
 inline void vol_shade_all(const DeviceScene &S, PathBufs &P, int cur, int grid, hipStream_t s, bool sph, bool basic) {
     if (P.vol_flight) {
-        hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, P.ctr, C_FLQ, 2);
-        hipLaunchKernelGGL(k_vol_flight_queue, dim3(std::max(1, grid / 4)), dim3(1024), 0, s, P, cur);
-        if (sph) hipLaunchKernelGGL(k_vol_flight<true>, dim3(grid), dim3(256), 0, s, S, P);
-        else hipLaunchKernelGGL(k_vol_flight<false>, dim3(grid), dim3(256), 0, s, S, P);
+        if (sph) hipLaunchKernelGGL(k_vol_flight<true>, dim3(grid), dim3(256), 0, s, S, P, cur);
+        else hipLaunchKernelGGL(k_vol_flight<false>, dim3(grid), dim3(256), 0, s, S, P, cur);
         vol_launch_check();
     }
     if (basic) {
@@ -751,21 +691,21 @@ inline void vol_shade_all(const DeviceScene &S, PathBufs &P, int cur, int grid, 
     vol_launch_check();
 }
 
-inline void vol_shadow(const DeviceScene &S, PathBufs &P, int grid, hipStream_t s, bool stats, bool sph) {
+inline void vol_shadow(const DeviceScene &S, PathBufs &P, int cur, int grid, hipStream_t s, bool stats, bool sph) {
     if (stats) {
-        if (sph) hipLaunchKernelGGL((k_vol_occlude<true, true>), dim3(grid), dim3(256), 0, s, S, P);
-        else hipLaunchKernelGGL((k_vol_occlude<true, false>), dim3(grid), dim3(256), 0, s, S, P);
+        if (sph) hipLaunchKernelGGL((k_vol_occlude<true, true>), dim3(grid), dim3(256), 0, s, S, P, cur);
+        else hipLaunchKernelGGL((k_vol_occlude<true, false>), dim3(grid), dim3(256), 0, s, S, P, cur);
     } else {
-        if (sph) hipLaunchKernelGGL((k_vol_occlude<false, true>), dim3(grid), dim3(256), 0, s, S, P);
-        else hipLaunchKernelGGL((k_vol_occlude<false, false>), dim3(grid), dim3(256), 0, s, S, P);
+        if (sph) hipLaunchKernelGGL((k_vol_occlude<false, true>), dim3(grid), dim3(256), 0, s, S, P, cur);
+        else hipLaunchKernelGGL((k_vol_occlude<false, false>), dim3(grid), dim3(256), 0, s, S, P, cur);
     }
     vol_launch_check();
     if (stats) {
-        if (sph) hipLaunchKernelGGL((k_vol_shadow<true, true>), dim3(grid), dim3(256), 0, s, S, P);
-        else hipLaunchKernelGGL((k_vol_shadow<true, false>), dim3(grid), dim3(256), 0, s, S, P);
+        if (sph) hipLaunchKernelGGL((k_vol_shadow<true, true>), dim3(grid), dim3(256), 0, s, S, P, cur);
+        else hipLaunchKernelGGL((k_vol_shadow<true, false>), dim3(grid), dim3(256), 0, s, S, P, cur);
     } else {
-        if (sph) hipLaunchKernelGGL((k_vol_shadow<false, true>), dim3(grid), dim3(256), 0, s, S, P);
-        else hipLaunchKernelGGL((k_vol_shadow<false, false>), dim3(grid), dim3(256), 0, s, S, P);
+        if (sph) hipLaunchKernelGGL((k_vol_shadow<false, true>), dim3(grid), dim3(256), 0, s, S, P, cur);
+        else hipLaunchKernelGGL((k_vol_shadow<false, false>), dim3(grid), dim3(256), 0, s, S, P, cur);
     }
     vol_launch_check();
 }
