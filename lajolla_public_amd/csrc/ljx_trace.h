@@ -208,7 +208,7 @@ struct TraceScene {
     const int8_t *__restrict__ skip = nullptr;  // OPAQUE traversals: per slot, nonzero to pass through
 };
 
-// Traversal state of one ray, advanced one inner node or one leaf per step.
+// Traversal state of one ray, advanced one inner node or one primitive per step.
 // stack: this lane's LDS column base (entries at stack[k*stride]); spill:
 // this lane's global spill column.  SPH: the scene has sphere primitives
 // (otherwise every leaf slot is a triangle).  OPAQUE (any hit only): slots
@@ -237,8 +237,10 @@ struct Tracer {
         hit.slot = -1;
     }
 
-    // One inner node or one leaf.  Returns true when the ray is finished: the
-    // stack ran empty, or (any hit) an occluder was found.
+    // One inner node or one primitive of a leaf, whichever phase the wave's
+    // calling lanes take; a ray in the other phase stays where it is.  Returns
+    // true when the ray is finished: the stack ran empty, or (any hit) an
+    // occluder was found.
     __device__ __forceinline__ bool step(const TraceScene &ts, int *stack, int stride, int *spill, int spill_stride,
                                          uint32_t &n_nodes, uint32_t &n_prims) {
         const float kMiss = __builtin_huge_valf();
@@ -253,7 +255,18 @@ struct Tracer {
             ca = k0;
             cb = k1;
         };
-        if (node >= 0) {
+        // One phase per step for the whole wave: rays at a node and rays at a
+        // leaf executed in turn leave two thirds of the lanes idle in each.
+        // A leaf's primitive costs about half a node's boxes and slabs, and
+        // shortens the ray, so leaves go first once half as many rays wait
+        // there.  Against both phases in every step: any hits of the 1080p
+        // terrain 27.6 -> 24.1 ms, closest hits 56.4 -> 53.7, of the nested
+        // media 76.8 -> 69.8 (inner nodes first for 1 : 1, 3 : 1 and 1 : 2
+        // rays: 56.1, 53.5, 59.9 and 70.9, 70.7, 73.8).
+        const bool inner = node >= 0;
+        const int at_node = __popcll(__ballot(inner)), at_leaf = __popcll(__ballot(!inner));
+        if (at_node >= 2 * at_leaf) {
+            if (!inner) return false;
             const Bvh4QNode *nd = ts.nodes + node;
             const float4 org = nd->org;
             const uint4 qx = nd->qx, qy = nd->qy, qz = nd->qz;
@@ -324,35 +337,38 @@ struct Tracer {
                 }
             }
         } else {
+            if (inner) return false;
+            // one primitive of the leaf
             const int code = ~node;
-            const int first = code >> 3, cnt = (code & 7) + 1;
-            for (int k = 0; k < cnt; k++) {
-                const int slot = first + k;
-                float4 p0 = ts.prims[3 * slot], p1 = ts.prims[3 * slot + 1];
-                float t, u = 0, v = 0;
-                bool ok;
-                if (STATS) n_prims++;
-                if (!SPH || __float_as_int(p1.w) == kPrimTri) {
-                    float4 p2 = ts.prims[3 * slot + 2];
-                    ok = tri_test(r, p0, p1, p2, tmin, tmax, t, u, v);
-                } else {
-                    double td;
-                    ok = sphere_roots(r.ox, r.oy, r.oz, dx, dy, dz, ts.spheres[__float_as_int(p1.x)], tmin, tmax, td);
-                    t = float(td);
-                }
-                if (OPAQUE && ok && ts.skip[slot]) {
-                    ok = false;
-                    passed = true;
-                }
-                if (ok) {
-                    found = true;
-                    hit.t = t;
-                    hit.u = u;
-                    hit.v = v;
-                    hit.slot = slot;
-                    if (ANY) return true;
-                    tmax = t;
-                }
+            const int slot = code >> 3;
+            float4 p0 = ts.prims[3 * slot], p1 = ts.prims[3 * slot + 1];
+            float t, u = 0, v = 0;
+            bool ok;
+            if (STATS) n_prims++;
+            if (!SPH || __float_as_int(p1.w) == kPrimTri) {
+                float4 p2 = ts.prims[3 * slot + 2];
+                ok = tri_test(r, p0, p1, p2, tmin, tmax, t, u, v);
+            } else {
+                double td;
+                ok = sphere_roots(r.ox, r.oy, r.oz, dx, dy, dz, ts.spheres[__float_as_int(p1.x)], tmin, tmax, td);
+                t = float(td);
+            }
+            if (OPAQUE && ok && ts.skip[slot]) {
+                ok = false;
+                passed = true;
+            }
+            if (ok) {
+                found = true;
+                hit.t = t;
+                hit.u = u;
+                hit.v = v;
+                hit.slot = slot;
+                if (ANY) return true;
+                tmax = t;
+            }
+            if (code & 7) {
+                node = ~(code + 8 - 1);  // the next slot, one primitive fewer
+                return false;
             }
         }
         if (sp == 0) return true;

@@ -140,3 +140,18 @@ def test_terrain_spheres_hit_parity(n_rays):
     assert agree.all(), np.nonzero(~agree)[0][:10]
     # and the oracle's any hit is the closest hit's verdict
     assert np.array_equal(occ_r[~ambiguous], (hit & (r["t"] <= tfar))[~ambiguous])
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 130, 4097])
+def test_rays_are_independent_of_their_wave(n):
+    """A ray's hit does not depend on the rays that share its wave (nodes and leaves are taken in phases that the
+    wave's rays choose together), whatever part of the wave is filled."""
+    desc = scenes.nested_media(seed=11, sphere_res=40)
+    sc = api.Scene(desc)
+    o, d = hit_parity_rays(desc, 5000, seed=3, bounds=sc.bounds())
+    hits, occ = hits_to_numpy(sc.trace_closest(make_rays(o, d))), np.asarray(sc.trace_any(make_rays(o, d)))
+    pick = np.random.default_rng(n).permutation(5000)[:n]
+    part = hits_to_numpy(sc.trace_closest(make_rays(o[pick], d[pick])))
+    for k in hits:
+        assert np.array_equal(hits[k][pick], part[k]), k
+    assert np.array_equal(occ[pick], np.asarray(sc.trace_any(make_rays(o[pick], d[pick]))))
