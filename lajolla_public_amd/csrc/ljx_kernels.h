@@ -28,9 +28,10 @@ namespace ljx {
 
 constexpr int kNumMatTypes = 9;
 constexpr int kBucketAny = 9;  // unsorted hits (below the sort threshold), shaded by runtime dispatch
-constexpr int kBucketMiss = 10;
-constexpr int kBucketNoMat = 11;
-constexpr int kNumBuckets = 12;
+constexpr int kBucketScatter = 10;  // volumetric paths that scatter in their medium
+constexpr int kBucketMiss = 11;     // buckets from here on cast no shadow rays
+constexpr int kBucketNoMat = 12;
+constexpr int kNumBuckets = 13;
 // counter slots
 constexpr int C_EXT = 0;      // C_EXT + (0|1): extension queues
 constexpr int C_BUCKET = 4;   // C_BUCKET + bucket: its paths
@@ -124,8 +125,8 @@ struct PathBufs {
     long long valid0;
 };
 
-// A vertex's shadow ray is written at its path's place in P.order (volumetric:
-// in the extension queue); places without one carry this mark in sh_occ.
+// A vertex's shadow ray is written at its path's place in P.order; places
+// without one carry this mark in sh_occ.
 constexpr uint8_t kShNone = 3;
 // Shadow-queue entries carry the path slot in the low kSlotBits bits and the
 // vertex index in the rest (clamped there: only the guiding record, a few

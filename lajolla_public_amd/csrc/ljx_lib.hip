@@ -1063,23 +1063,33 @@ void launch(K kernel, int grid, int block, hipStream_t s, A... args) {
 // they run on three streams at once: a long kernel at one wave per SIMD
 // (DisneyBSDF) leaves most of each SIMD to the others, and the launches'
 // tails overlap.  Captured work (batches) keeps them on one stream.
+void fan_out(Scene &sc, hipStream_t s, bool fan, hipStream_t (&st)[3]) {
+    st[0] = st[1] = st[2] = s;
+    if (!fan) return;
+    for (int k = 0; k < 2; k++) {
+        if (!sc.side[k]) HIPX(hipStreamCreateWithFlags(&sc.side[k], hipStreamNonBlocking));
+        if (!sc.ev_join[k]) HIPX(hipEventCreateWithFlags(&sc.ev_join[k], hipEventDisableTiming));
+    }
+    if (!sc.ev_fork) HIPX(hipEventCreateWithFlags(&sc.ev_fork, hipEventDisableTiming));
+    HIPX(hipEventRecord(sc.ev_fork, s));
+    for (int k = 0; k < 2; k++) {
+        HIPX(hipStreamWaitEvent(sc.side[k], sc.ev_fork, 0));
+        st[k + 1] = sc.side[k];
+    }
+}
+void fan_in(Scene &sc, hipStream_t s, bool fan) {
+    if (!fan) return;
+    for (int k = 0; k < 2; k++) {
+        HIPX(hipEventRecord(sc.ev_join[k], sc.side[k]));
+        HIPX(hipStreamWaitEvent(s, sc.ev_join[k], 0));
+    }
+}
 template <bool SPH, bool GUIDE>
 void shade_all_t(Scene &sc, PathBufs &P, int cur, int grid, int block, hipStream_t s, bool fan) {
     const DeviceScene &S = sc.ds;
     unsigned m = sc.mat_types_present;
-    hipStream_t st[3] = {s, s, s};
-    if (fan) {
-        for (int k = 0; k < 2; k++) {
-            if (!sc.side[k]) HIPX(hipStreamCreateWithFlags(&sc.side[k], hipStreamNonBlocking));
-            if (!sc.ev_join[k]) HIPX(hipEventCreateWithFlags(&sc.ev_join[k], hipEventDisableTiming));
-        }
-        if (!sc.ev_fork) HIPX(hipEventCreateWithFlags(&sc.ev_fork, hipEventDisableTiming));
-        HIPX(hipEventRecord(sc.ev_fork, s));
-        for (int k = 0; k < 2; k++) {
-            HIPX(hipStreamWaitEvent(sc.side[k], sc.ev_fork, 0));
-            st[k + 1] = sc.side[k];
-        }
-    }
+    hipStream_t st[3];
+    fan_out(sc, s, fan, st);
     int next = 0;
     auto on = [&]() { return st[next++ % 3]; };
     // the heaviest kernels first, one per stream
@@ -1095,12 +1105,7 @@ void shade_all_t(Scene &sc, PathBufs &P, int cur, int grid, int block, hipStream
     // unsorted bounces and textured materials go to the runtime-dispatch kernel
     if (P.sort_threshold > 0 || sc.has_textured) launch(k_shade<-1, SPH, GUIDE>, grid, block, on(), S, P, cur);
     launch(k_miss, grid, block, on(), S, P);
-    if (fan) {
-        for (int k = 0; k < 2; k++) {
-            HIPX(hipEventRecord(sc.ev_join[k], sc.side[k]));
-            HIPX(hipStreamWaitEvent(s, sc.ev_join[k], 0));
-        }
-    }
+    fan_in(sc, s, fan);
 }
 void shade_all(Scene &sc, PathBufs &P, int cur, int grid, hipStream_t s, bool guide, int block = 256,
                bool fan = false) {
@@ -1144,6 +1149,16 @@ void sort_ext_queue(PathBufs &P, int n, int cur, hipStream_t s) {
     launch(k_sort_count, nblk, 256, s, P, cur, nblk);
     launch(k_sort_scan, kNumBuckets, 1024, s, P, cur, nblk);
     launch(k_sort_scatter, nblk, 256, s, P, cur, nblk);
+}
+
+// A volumetric bounce between its closest hits and its shadow walks.
+void vol_stage(Scene &sc, PathBufs &P, int n, int cur, int grid, hipStream_t s, bool fan) {
+    vol_events(sc.ds, P, cur, grid, s, sc.has_spheres);
+    sort_ext_queue(P, n, cur, s);
+    hipStream_t st[3];
+    fan_out(sc, s, fan, st);
+    vol_shade_all(sc.ds, P, cur, grid, st, sc.has_spheres, (sc.mat_types_present & ~7u) == 0);
+    fan_in(sc, s, fan);
 }
 
 void trace_stage(Scene &sc, PathBufs &P, int cur, int grid, int sgrid, hipStream_t s, bool stats, bool shadow) {
@@ -1374,12 +1389,12 @@ void render_impl(Scene &sc, const ljx_render_options *o, const ljx_exec_options 
                     tm.end(4, ev);
                 }
                 tm.begin(2, ev);
-                if (vol) vol_shade_all(S, P, cur, shade_grid, s, sc.has_spheres, (sc.mat_types_present & ~7u) == 0);
+                if (vol) vol_stage(sc, P, ns * nq, cur, shade_grid, s, /*fan=*/true);
                 else shade_all(sc, P, cur, shade_grid, s, guided, shade_block, /*fan=*/true);
                 build_ext_queue(P, ns * nq, cur, s);
                 tm.end(2, ev);
                 tm.begin(1, ev);
-                if (vol) vol_shadow(S, P, cur, tgrid, s, stats_on, sc.has_spheres);
+                if (vol) vol_shadow(S, P, tgrid, s, stats_on, sc.has_spheres);
                 else trace_stage(sc, P, cur, tgrid, shade_grid, s, stats_on, true);
                 tm.end(1, ev);
                 cur ^= 1;
@@ -1694,10 +1709,10 @@ void batch_impl(const ljx_batch_job *jobs, size_t njobs, const ljx_exec_options 
                 for (int b = 0; b < std::max(P.max_depth, 1); b++) {
                     trace_stage(sc, P, cur, tgrid, sgrid, cs, false, false);
                     if (!vol) sort_ext_queue(P, n, cur, cs);
-                    if (vol) vol_shade_all(S, P, cur, sgrid, cs, sc.has_spheres, (sc.mat_types_present & ~7u) == 0);
+                    if (vol) vol_stage(sc, P, n, cur, sgrid, cs, /*fan=*/false);
                     else shade_all(sc, P, cur, sgrid, cs, false, gp.block);
                     build_ext_queue(P, n, cur, cs);
-                    if (vol) vol_shadow(S, P, cur, tgrid, cs, false, sc.has_spheres);
+                    if (vol) vol_shadow(S, P, tgrid, cs, false, sc.has_spheres);
                     else trace_stage(sc, P, cur, tgrid, sgrid, cs, false, true);
                     cur ^= 1;
                 }

@@ -11,9 +11,10 @@
 // max_null_collisions cap (:760-764).
 //
 //   k_vol_flight  free flight (delta tracking) in scenes with grid media
-//   k_vol_shade   free flight in homogeneous media, emission with MIS,
-//                 index-matched pass-through, phase or BSDF sampling, NEE
-//                 light-point sampling, RR
+//   k_vol_event   whether a path scatters before its hit, in scenes without
+//   k_sort_*      orders the paths by what happens to them
+//   k_vol_shade   by event: phase or BSDF sampling, NEE light-point sampling,
+//                 RR, emission with MIS, index-matched pass-through
 //   k_vol_shadow  the NEE shadow walk: closest hits through index-matched
 //                 surfaces with ratio tracking in every medium on the way
 //
@@ -66,8 +67,9 @@ __device__ __forceinline__ int update_medium(D3 dir, const Vertex &v, int medium
 // tracking; its first draw picks the channel).  It is the first use of the
 // path's stream in a bounce, so in scenes with grid media (long loops of
 // null collisions) k_vol_flight runs it for every path of the queue before
-// k_vol_shade, which takes over the stream state; otherwise k_vol_shade runs
-// it in place.
+// k_vol_shade, which takes over the stream state; in homogeneous media (one
+// collision) k_vol_event runs it to learn the outcome and k_vol_shade again,
+// which is cheaper than 128 bytes of FP64 results written and read.
 struct Flight {
     D3 T, trans_dir_pdf;
     double accum_t;
@@ -96,8 +98,11 @@ __device__ __forceinline__ void flight_begin(FlightRun &r, const DeviceScene &S,
     r.ch = min(max(int(u * 3), 0), 2);
     r.it = 0;
 }
-// One pass of the loop; true when the flight has ended.
-__device__ __forceinline__ bool flight_step(FlightRun &r, const PathBufs &P, uint64_t &st, uint64_t inc) {
+// One pass of the loop; true when the flight has ended.  decided: whether the
+// path collides before its hit, where an earlier kernel has found that out (1
+// or 0, else -1): two compilations of the comparison may round differently.
+__device__ __forceinline__ bool flight_step(FlightRun &r, const PathBufs &P, uint64_t &st, uint64_t inc,
+                                            int decided = -1) {
     Flight &fl = r.fl;
     const D3 maj = r.maj;
     const double max_maj = r.max_maj;
@@ -108,7 +113,7 @@ __device__ __forceinline__ bool flight_step(FlightRun &r, const PathBufs &P, uin
     const double t = -log(1 - pcg_double(st, inc)) / mc;
     const double dt = r.t_hit - fl.accum_t;
     fl.accum_t = fmin(fl.accum_t + t, r.t_hit);
-    if (t < dt) {
+    if (decided < 0 ? t < dt : decided > 0) {
         D3 sig_t = sigma_t_at(*r.m, r.org + fl.accum_t * r.dir);
         D3 real_prob = sig_t / maj;
         D3 e = maj_exp(maj, r.grey, t);
@@ -130,10 +135,10 @@ __device__ __forceinline__ bool flight_step(FlightRun &r, const PathBufs &P, uin
     return true;
 }
 __device__ __forceinline__ Flight free_flight(const DeviceScene &S, const PathBufs &P, int medium, D3 org, D3 dir,
-                                              double t_hit, uint64_t &st, uint64_t inc) {
+                                              double t_hit, uint64_t &st, uint64_t inc, int decided = -1) {
     FlightRun r;
     flight_begin(r, S, medium, org, dir, t_hit, st, inc);
-    while (!flight_step(r, P, st, inc)) {
+    while (!flight_step(r, P, st, inc, decided)) {
     }
     return r.fl;
 }
@@ -148,6 +153,31 @@ __device__ __forceinline__ double hit_distance(const DeviceScene &S, float4 h, D
     return sqrt(dist2(org, v.pos));
 }
 
+// The bucket of a path: scattered in its medium, or the hit's (k_extend).
+__device__ __forceinline__ uint8_t event_bucket(const DeviceScene &S, bool scatter, float4 hit) {
+    const int slot = __float_as_int(hit.w);
+    return uint8_t(scatter ? kBucketScatter : slot < 0 ? kBucketMiss : S.slot_bucket[slot]);
+}
+template <bool SPH>
+__global__ __launch_bounds__(256) void k_vol_event(DeviceScene S, PathBufs P, int cur) {
+    const uint32_t *q = cur ? P.extq1 : P.extq0;
+    const int n = P.ctr[C_EXT + cur];
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const uint32_t pid = q[i];
+        const float4 h = P.hit[pid];
+        const int medium = P.medium[pid];
+        bool scatter = false;
+        if (medium >= 0) {
+            const float4 ro = P.ray_o[pid], rd = P.ray_d[pid];
+            const D3 org = f3d(ro), dir = f3d(rd);
+            uint64_t st = P.rng[pid];
+            const uint64_t inc = pcg_inc(slot_info(P, int(pid)).stream());
+            scatter = free_flight(S, P, medium, org, dir, hit_distance<SPH>(S, h, org, dir), st, inc).scatter;
+        }
+        P.key[i] = event_bucket(S, scatter, h);
+    }
+}
+
 // Free flight for the queue's paths that are in a medium, in a kernel small
 // enough for three waves per SIMD.  The loops' lengths vary widely between
 // paths, so a lane whose flight ended (or whose path is in no medium) takes
@@ -160,6 +190,7 @@ __global__ __launch_bounds__(256) void k_vol_flight(DeviceScene S, PathBufs P, i
     FlightRun r;
     uint64_t st = 0, inc = 0;
     uint32_t pid = 0;
+    int i = 0;
     bool busy = false, fin = false;
     FeedRange range;
     range.start(P.ctr + C_FEED_FLIGHT, P.ctr[C_EXT + cur], kFeedTickets);
@@ -172,10 +203,17 @@ __global__ __launch_bounds__(256) void k_vol_flight(DeviceScene S, PathBufs P, i
                 P.vf_t[pid] = make_double4(r.fl.T.x, r.fl.T.y, r.fl.T.z, r.fl.accum_t);
                 P.vf_p[pid] = make_double4(r.fl.trans_dir_pdf.x, r.fl.trans_dir_pdf.y, r.fl.trans_dir_pdf.z,
                                            r.fl.scatter ? 1.0 : 0.0);
+                P.key[i] = event_bucket(S, r.fl.scatter, P.hit[pid]);
                 fin = false;
             }
-            const int i = range.take(!busy, [&](int j) { return P.medium[q[j]] >= 0; });
-            if (i >= 0) {
+            const int k = range.take(!busy, [&](int j) {
+                const uint32_t p = q[j];
+                const bool in_medium = P.medium[p] >= 0;
+                if (!in_medium) P.key[j] = event_bucket(S, false, P.hit[p]);
+                return in_medium;
+            });
+            if (k >= 0) {
+                i = k;
                 pid = q[i];
                 const float4 ro = P.ray_o[pid], rd = P.ray_d[pid];
                 const D3 org = f3d(ro), dir = f3d(rd);
@@ -193,40 +231,41 @@ __global__ __launch_bounds__(256) void k_vol_flight(DeviceScene S, PathBufs P, i
     }
 }
 
-template <bool SPH, int DMT>
+// What happens to a path at the end of its flight, by bucket.  One kernel for
+// all of them ran with 30 of 64 lanes active, one wave per SIMD and every
+// field of the state read and written whatever the event; by event the kernels
+// move only what theirs needs (scattering: no hit, vertex, radiance or MIS
+// caches) and nothing for paths that left the scene: 126 -> 75 ms for the
+// 1024x1024 128-sample nested media with k_vol_event and the sort.
+constexpr int kEvScatter = 0, kEvSurface = 1, kEvPass = 2;
+template <bool SPH, int DMT, int EV>
 __device__ __forceinline__ void vol_shade(const DeviceScene &S, const PathBufs &P, uint32_t pid, bool &push_ext,
                                           bool &push_sh, float4 &sh_o, float4 &sh_d, float4 &sh_c, float4 &sh_x) {
-    float4 h = P.hit[pid];
+    constexpr bool scatter = EV == kEvScatter;
+    push_ext = false;
+    push_sh = false;
     float4 ro = P.ray_o[pid], rd = P.ray_d[pid];
     D3 org = f3d(ro), dir = f3d(rd);
     int bounces = P.depth[pid];
+    // a path at the last depth may still reach a light
+    const bool last = P.max_depth != -1 && bounces == P.max_depth - 1;
+    if (scatter && last) return;
     uint64_t st = P.rng[pid];
     const uint64_t stream = slot_info(P, int(pid)).stream();
     uint64_t inc = pcg_inc(stream);
     float4 tp4 = P.tp[pid];
     D3 tp{tp4.x, tp4.y, tp4.z};
     double eta_scale = tp4.w;
-    float4 r4 = P.rad[pid];
-    D3 rad{r4.x, r4.y, r4.z};
     int medium = P.medium[pid];
-    float4 nc = P.nee_c[pid];
-    D3 nee_p_cache{nc.x, nc.y, nc.z};
-    double dir_pdf = nc.w;
-    float4 mt = P.mtp[pid];
-    D3 multi_trans_pdf{mt.x, mt.y, mt.z};
-    bool never_scatter = mt.w != 0.f;
-    push_ext = false;
-    push_sh = false;
 
-    int slot = __float_as_int(h.w);
-    bool hit = slot >= 0;
     Vertex v;
-    if (hit) v = make_vertex<SPH>(S, slot, h.x, h.y, h.z, org, dir);
-    bool scatter = false;
-    bool alive = true;
-    D3 p_scatter = org;
+    if constexpr (!scatter) {
+        const float4 h = P.hit[pid];
+        v = make_vertex<SPH>(S, __float_as_int(h.w), h.x, h.y, h.z, org, dir);
+    }
+    D3 p_scatter = org, trans_dir_pdf{1, 1, 1};
     if (medium >= 0) {
-        D3 T, trans_dir_pdf;
+        D3 T;
         double accum_t;
         if (P.vol_flight) {
             // the free flight k_vol_flight sampled (it advanced the stream state)
@@ -234,56 +273,61 @@ __device__ __forceinline__ void vol_shade(const DeviceScene &S, const PathBufs &
             T = D3{ft.x, ft.y, ft.z};
             trans_dir_pdf = D3{fp.x, fp.y, fp.z};
             accum_t = ft.w;
-            scatter = fp.w != 0.0;
         } else {
-            const Flight fl = free_flight(S, P, medium, org, dir, hit ? sqrt(dist2(org, v.pos)) : __builtin_huge_val(),
-                                          st, inc);
+            const Flight fl = free_flight(S, P, medium, org, dir,
+                                          scatter ? __builtin_huge_val() : sqrt(dist2(org, v.pos)), st, inc, scatter);
             T = fl.T;
             trans_dir_pdf = fl.trans_dir_pdf;
             accum_t = fl.accum_t;
-            scatter = fl.scatter;
         }
-        if (scatter) never_scatter = false;
-        if (isfinite(accum_t)) p_scatter = org + accum_t * dir;
-        multi_trans_pdf = multi_trans_pdf * trans_dir_pdf;
+        if (scatter) p_scatter = org + accum_t * dir;
         tp = tp * T / avgc(trans_dir_pdf);
     }
-    if (!scatter && !hit) alive = false;
-    if (alive && !scatter && v.area_light_id >= 0) {
-        const LightRec &l = S.lights[v.area_light_id];
-        LightPoint lp{v.pos, v.g.ng};
-        D3 Le = light_emission(S, l, -dir, lp);
-        if (never_scatter) {
-            rad = rad + tp * Le;
-        } else {
-            double pdf_nee = S.light_pmf[v.area_light_id] * pdf_light_point(S, l, lp, nee_p_cache);
-            double G = fabs(dot(dir, v.g.ng)) / dist2(nee_p_cache, v.pos);
-            double dp = dir_pdf * avgc(multi_trans_pdf) * G;
-            double w = (dp * dp) / (dp * dp + pdf_nee * pdf_nee);
-            rad = rad + tp * Le * w;
+    if constexpr (!scatter) {
+        if (v.area_light_id >= 0) {
+            const LightRec &l = S.lights[v.area_light_id];
+            LightPoint lp{v.pos, v.g.ng};
+            D3 add = tp * light_emission(S, l, -dir, lp);
+            const float4 mt = P.mtp[pid];
+            if (mt.w == 0.f) {  // some vertex of the path scattered
+                const float4 nc = P.nee_c[pid];
+                const D3 nee_p_cache{nc.x, nc.y, nc.z};
+                const D3 multi_trans_pdf = D3{mt.x, mt.y, mt.z} * trans_dir_pdf;
+                double pdf_nee = S.light_pmf[v.area_light_id] * pdf_light_point(S, l, lp, nee_p_cache);
+                double G = fabs(dot(dir, v.g.ng)) / dist2(nee_p_cache, v.pos);
+                double dp = double(nc.w) * avgc(multi_trans_pdf) * G;
+                add = add * ((dp * dp) / (dp * dp + pdf_nee * pdf_nee));
+            }
+            const float4 r4 = P.rad[pid];
+            P.rad[pid] = make_float4(float(r4.x + add.x), float(r4.y + add.y), float(r4.z + add.z), 0.f);
         }
+        if (last) return;
     }
-    if (alive && P.max_depth != -1 && bounces == P.max_depth - 1) alive = false;
-    bool passed = false;
-    if (alive && !scatter && v.material_id == -1) {
+    if constexpr (EV == kEvPass) {
         // index-matched interface: continue straight through
-        medium = update_medium(dir, v, medium);
+        const float4 mt = P.mtp[pid];
+        const D3 multi_trans_pdf = D3{mt.x, mt.y, mt.z} * trans_dir_pdf;
         P.ray_o[pid] = make_float4(float(v.pos.x), float(v.pos.y), float(v.pos.z), float(S.eps));
         P.ray_d[pid] = make_float4(float(dir.x), float(dir.y), float(dir.z), __builtin_huge_valf());
-        bounces++;
+        P.depth[pid] = bounces + 1;
+        if (!P.vol_flight) P.rng[pid] = st;
+        P.medium[pid] = update_medium(dir, v, medium);
+        P.tp[pid] = make_float4(float(tp.x), float(tp.y), float(tp.z), float(eta_scale));
+        P.mtp[pid] = make_float4(float(multi_trans_pdf.x), float(multi_trans_pdf.y), float(multi_trans_pdf.z), mt.w);
         push_ext = true;
-        passed = true;
-    }
-    if (alive && !passed) {
+        return;
+    } else {
         D3 dir_view = -dir;
         // NEE sub-stream
         uint32_t k = pcg_next(st, inc);
         uint64_t nstream = stream ^ kNeeStreamXor;
         uint64_t ninc = pcg_inc(nstream);
         uint64_t nst = pcg_init_state(nstream, uint64_t(k));
-        D3 pos = scatter ? p_scatter : v.pos;
+        const D3 pos = scatter ? p_scatter : v.pos;
         double lu0 = pcg_double(nst, ninc), lu1 = pcg_double(nst, ninc);
         double lw = pcg_double(nst, ninc), sw = pcg_double(nst, ninc);
+        D3 sigma_s{0, 0, 0};
+        if (scatter) sigma_s = sigma_s_at(S.media[medium], p_scatter);
         if (S.num_lights > 0) {
             int lid = sample_cdf_guided(S.light_cdf, S.num_lights, lw, S.light_guide, S.light_guide_m);
             const LightRec &l = S.lights[lid];
@@ -295,12 +339,11 @@ __device__ __forceinline__ void vol_shade(const DeviceScene &S, const PathBufs &
                 D3 f;
                 double pdf_f;
                 D3 pre = tp;
-                if (scatter) {
-                    const MediumRec &m = S.media[medium];
-                    double pv = phase_value(m, dir_view, dir_light);
+                if constexpr (scatter) {
+                    double pv = phase_value(S.media[medium], dir_view, dir_light);
                     f = D3{pv, pv, pv};
                     pdf_f = pv;
-                    pre = pre * sigma_s_at(m, p_scatter);
+                    pre = pre * sigma_s;
                 } else {
                     MatRec mat = S.materials[v.material_id];
                     if (mat.textured) resolve_textures(S, mat, v.tu, v.tv, 0.0);
@@ -319,87 +362,71 @@ __device__ __forceinline__ void vol_shade(const DeviceScene &S, const PathBufs &
                 }
             }
         }
-        if (scatter) {
+        double dir_pdf;
+        D3 next_dir;
+        float tnear;
+        if constexpr (scatter) {
             const MediumRec &m = S.media[medium];
             double u0 = pcg_double(st, inc), u1 = pcg_double(st, inc);
-            D3 nd = phase_sample(m, dir_view, u0, u1);
-            double pv = phase_value(m, dir_view, nd);
-            if (pv <= 0) {
-                alive = false;
-            } else {
-                tp = tp * (D3{pv, pv, pv} / pv) * sigma_s_at(m, p_scatter);
-                dir_pdf = pv;
-                nee_p_cache = p_scatter;
-                multi_trans_pdf = D3{1, 1, 1};
-                P.ray_o[pid] = make_float4(float(p_scatter.x), float(p_scatter.y), float(p_scatter.z), 0.f);
-                P.ray_d[pid] = make_float4(float(nd.x), float(nd.y), float(nd.z), __builtin_huge_valf());
-            }
+            next_dir = phase_sample(m, dir_view, u0, u1);
+            dir_pdf = phase_value(m, dir_view, next_dir);
+            if (dir_pdf <= 0) return;
+            tp = tp * (D3{dir_pdf, dir_pdf, dir_pdf} / dir_pdf) * sigma_s;
+            tnear = 0.f;
         } else {
             MatRec mat = S.materials[v.material_id];
             if (mat.textured) resolve_textures(S, mat, v.tu, v.tv, 0.0);
             double u0 = pcg_double(st, inc), u1 = pcg_double(st, inc), w = pcg_double(st, inc);
             BsdfSample bs = bsdf_sample<DMT>(mat, dir_view, v.g, u0, u1, w);
-            if (!bs.valid) {
-                alive = false;
-            } else {
-                if (bs.eta != 0) eta_scale /= (bs.eta * bs.eta);
-                D3 f = bsdf_eval<DMT>(mat, dir_view, bs.dir, v.g);
-                double pdf = bsdf_pdf<DMT>(mat, dir_view, bs.dir, v.g);
-                if (pdf <= 0) {
-                    alive = false;
-                } else {
-                    tp = tp * f / pdf;
-                    dir_pdf = pdf;
-                    nee_p_cache = v.pos;
-                    multi_trans_pdf = D3{1, 1, 1};
-                    never_scatter = false;
-                    medium = update_medium(bs.dir, v, medium);
-                    P.ray_o[pid] = make_float4(float(v.pos.x), float(v.pos.y), float(v.pos.z), float(S.eps));
-                    P.ray_d[pid] = make_float4(float(bs.dir.x), float(bs.dir.y), float(bs.dir.z), __builtin_huge_valf());
-                }
-            }
+            if (!bs.valid) return;
+            if (bs.eta != 0) eta_scale /= (bs.eta * bs.eta);
+            D3 f = bsdf_eval<DMT>(mat, dir_view, bs.dir, v.g);
+            dir_pdf = bsdf_pdf<DMT>(mat, dir_view, bs.dir, v.g);
+            if (dir_pdf <= 0) return;
+            tp = tp * f / dir_pdf;
+            medium = update_medium(bs.dir, v, medium);
+            next_dir = bs.dir;
+            tnear = float(S.eps);
         }
-        if (alive && bounces >= P.rr_depth) {
+        if (bounces >= P.rr_depth) {
             double rr = fmin(maxc((1 / eta_scale) * tp), 0.95);
-            if (pcg_double(st, inc) > rr) alive = false;
-            else tp = tp / rr;
+            if (pcg_double(st, inc) > rr) return;
+            tp = tp / rr;
         }
-        if (alive) {
-            bounces++;
-            push_ext = true;
-        }
+        // a path that goes on; an ended one's state is not read again
+        push_ext = true;
+        P.ray_o[pid] = make_float4(float(pos.x), float(pos.y), float(pos.z), tnear);
+        P.ray_d[pid] = make_float4(float(next_dir.x), float(next_dir.y), float(next_dir.z), __builtin_huge_valf());
+        P.depth[pid] = bounces + 1;
+        P.rng[pid] = st;
+        if (!scatter) P.medium[pid] = medium;
+        P.tp[pid] = make_float4(float(tp.x), float(tp.y), float(tp.z), float(eta_scale));
+        P.nee_c[pid] = make_float4(float(pos.x), float(pos.y), float(pos.z), float(dir_pdf));
+        P.mtp[pid] = make_float4(1.f, 1.f, 1.f, 0.f);
     }
-    P.depth[pid] = bounces;
-    P.rng[pid] = st;
-    P.medium[pid] = medium;
-    P.tp[pid] = make_float4(float(tp.x), float(tp.y), float(tp.z), float(eta_scale));
-    P.rad[pid] = make_float4(float(rad.x), float(rad.y), float(rad.z), 0.f);
-    P.nee_c[pid] = make_float4(float(nee_p_cache.x), float(nee_p_cache.y), float(nee_p_cache.z), float(dir_pdf));
-    P.mtp[pid] = make_float4(float(multi_trans_pdf.x), float(multi_trans_pdf.y), float(multi_trans_pdf.z),
-                             never_scatter ? 1.f : 0.f);
 }
 
-template <bool SPH, int DMT>
+template <bool SPH, int DMT, int EV>
 __global__ __launch_bounds__(256) void k_vol_shade(DeviceScene S, PathBufs P, int cur) {
-    // paths decide between medium and surface events after free-flight
-    // sampling, so they are not sorted: the extension queue as it is
-    int n = P.ctr[C_EXT + cur];
-    const uint32_t *q = cur ? P.extq1 : P.extq0;
-    int stride = gridDim.x * blockDim.x;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const uint32_t pid = q[i];
-        bool pe = false, ps = false;
+    // surface buckets of all material types lie together
+    constexpr int first = EV == kEvScatter ? kBucketScatter : EV == kEvSurface ? 0 : kBucketNoMat;
+    constexpr int end = EV == kEvSurface ? kBucketScatter : first + 1;
+    const int j0 = bucket_start(P, first), j1 = bucket_start(P, end);
+    for (int j = j0 + blockIdx.x * blockDim.x + threadIdx.x; j < j1; j += gridDim.x * blockDim.x) {
+        const uint32_t pid = P.order[j];
+        bool pe, ps;
         float4 so, sd, sc, sx;
-        vol_shade<SPH, DMT>(S, P, pid, pe, ps, so, sd, sc, sx);
+        vol_shade<SPH, DMT, EV>(S, P, pid, pe, ps, so, sd, sc, sx);
         if (pe) P.alive[pid] = 1;
-        // the shadow ray takes its path's place in the queue (shade_queue):
-        // appending it took one of 11.3 ns after the other per wave
-        P.sh_occ[i] = ps ? uint8_t(0) : kShNone;
-        if (ps) {
-            P.sh_o[i] = so;
-            P.sh_d[i] = sd;
-            P.sh_c[i] = sc;
-            P.sh_x[i] = sx;
+        if constexpr (EV != kEvPass) {
+            // the shadow ray takes its path's place in the order (shade_queue)
+            P.sh_occ[j] = ps ? uint8_t(0) : kShNone;
+            if (ps) {
+                P.sh_o[j] = so;
+                P.sh_d[j] = sd;
+                P.sh_c[j] = sc;
+                P.sh_x[j] = sx;
+            }
         }
     }
 }
@@ -416,7 +443,7 @@ __global__ __launch_bounds__(256) void k_vol_shade(DeviceScene S, PathBufs P, in
 // waves per SIMD.  Triangle-only scenes cap it at eight waves per SIMD (64
 // registers, a 16-byte spill).
 template <bool STATS, bool SPH>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? 1 : 8))) void k_vol_occlude(DeviceScene S, PathBufs P, int cur) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? 1 : 8))) void k_vol_occlude(DeviceScene S, PathBufs P) {
     __shared__ int stack[kStackLds * 256];
     const TraceScene ts{S.qnodes, S.prims, S.spheres, S.slot_passthru};
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x;
@@ -426,7 +453,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? 1 : 8
     Tracer<true, STATS, SPH, true> tr;
     bool busy = false, fin = false;
     FeedRange range;
-    range.start(P.ctr + C_FEED_SHADOW, P.ctr[C_EXT + cur]);
+    range.start(P.ctr + C_FEED_SHADOW, bucket_start(P, kBucketMiss));
     int i = 0, rays = 0;
     while (true) {
         const uint64_t idle = __ballot(!busy);
@@ -565,7 +592,7 @@ __device__ __forceinline__ bool walk_advance(Walk &w, const PathBufs &P) {
 // 768x576 64-sample smoke render.
 constexpr int kWalkRefill = 16;
 template <bool STATS, bool SPH>
-__global__ __launch_bounds__(256) void k_vol_shadow(DeviceScene S, PathBufs P, int cur) {
+__global__ __launch_bounds__(256) void k_vol_shadow(DeviceScene S, PathBufs P) {
     __shared__ int stack[kStackLds * 256];
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x;
     const int stride = gridDim.x * blockDim.x;
@@ -577,7 +604,7 @@ __global__ __launch_bounds__(256) void k_vol_shadow(DeviceScene S, PathBufs P, i
     // a busy lane is at a segment's start (wait) or inside one
     bool busy = false, fin = false, wait = false;
     FeedRange range;
-    range.start(P.ctr + C_FEED_WALK, P.ctr[C_EXT + cur], kFeedTickets);
+    range.start(P.ctr + C_FEED_WALK, bucket_start(P, kBucketMiss), kFeedTickets);
     while (true) {
         const uint64_t idle = __ballot(!busy);
         const int nidle = __popcll(idle);
@@ -674,38 +701,49 @@ inline void vol_launch_check() {
     if (e != hipSuccess) throw std::runtime_error(std::string("volpath kernel launch: ") + hipGetErrorString(e));
 }
 
-// basic: the scene uses no material types beyond lajolla's three basic ones.
-inline void vol_shade_all(const DeviceScene &S, PathBufs &P, int cur, int grid, hipStream_t s, bool sph, bool basic) {
+// What happens to each path of the extension queue: free flight and the sort's keys.
+inline void vol_events(const DeviceScene &S, PathBufs &P, int cur, int grid, hipStream_t s, bool sph) {
     if (P.vol_flight) {
         if (sph) hipLaunchKernelGGL(k_vol_flight<true>, dim3(grid), dim3(256), 0, s, S, P, cur);
         else hipLaunchKernelGGL(k_vol_flight<false>, dim3(grid), dim3(256), 0, s, S, P, cur);
-        vol_launch_check();
-    }
-    if (basic) {
-        if (sph) hipLaunchKernelGGL((k_vol_shade<true, kMtBasic>), dim3(grid), dim3(256), 0, s, S, P, cur);
-        else hipLaunchKernelGGL((k_vol_shade<false, kMtBasic>), dim3(grid), dim3(256), 0, s, S, P, cur);
     } else {
-        if (sph) hipLaunchKernelGGL((k_vol_shade<true, -1>), dim3(grid), dim3(256), 0, s, S, P, cur);
-        else hipLaunchKernelGGL((k_vol_shade<false, -1>), dim3(grid), dim3(256), 0, s, S, P, cur);
+        if (sph) hipLaunchKernelGGL(k_vol_event<true>, dim3(grid), dim3(256), 0, s, S, P, cur);
+        else hipLaunchKernelGGL(k_vol_event<false>, dim3(grid), dim3(256), 0, s, S, P, cur);
     }
     vol_launch_check();
 }
+// The shading kernels, on the streams given (one may stand for all three).
+// basic: the scene uses no material types beyond lajolla's three basic ones.
+template <bool SPH>
+void vol_shade_t(const DeviceScene &S, PathBufs &P, int cur, int grid, const hipStream_t (&s)[3], bool basic) {
+    const dim3 g(grid), b(256);
+    if (basic) hipLaunchKernelGGL((k_vol_shade<SPH, kMtBasic, kEvSurface>), g, b, 0, s[0], S, P, cur);
+    else hipLaunchKernelGGL((k_vol_shade<SPH, -1, kEvSurface>), g, b, 0, s[0], S, P, cur);
+    hipLaunchKernelGGL((k_vol_shade<SPH, kMtBasic, kEvScatter>), g, b, 0, s[1], S, P, cur);
+    hipLaunchKernelGGL((k_vol_shade<SPH, kMtBasic, kEvPass>), g, b, 0, s[2], S, P, cur);
+    vol_launch_check();
+}
+inline void vol_shade_all(const DeviceScene &S, PathBufs &P, int cur, int grid, const hipStream_t (&s)[3], bool sph,
+                          bool basic) {
+    if (sph) vol_shade_t<true>(S, P, cur, grid, s, basic);
+    else vol_shade_t<false>(S, P, cur, grid, s, basic);
+}
 
-inline void vol_shadow(const DeviceScene &S, PathBufs &P, int cur, int grid, hipStream_t s, bool stats, bool sph) {
+inline void vol_shadow(const DeviceScene &S, PathBufs &P, int grid, hipStream_t s, bool stats, bool sph) {
     if (stats) {
-        if (sph) hipLaunchKernelGGL((k_vol_occlude<true, true>), dim3(grid), dim3(256), 0, s, S, P, cur);
-        else hipLaunchKernelGGL((k_vol_occlude<true, false>), dim3(grid), dim3(256), 0, s, S, P, cur);
+        if (sph) hipLaunchKernelGGL((k_vol_occlude<true, true>), dim3(grid), dim3(256), 0, s, S, P);
+        else hipLaunchKernelGGL((k_vol_occlude<true, false>), dim3(grid), dim3(256), 0, s, S, P);
     } else {
-        if (sph) hipLaunchKernelGGL((k_vol_occlude<false, true>), dim3(grid), dim3(256), 0, s, S, P, cur);
-        else hipLaunchKernelGGL((k_vol_occlude<false, false>), dim3(grid), dim3(256), 0, s, S, P, cur);
+        if (sph) hipLaunchKernelGGL((k_vol_occlude<false, true>), dim3(grid), dim3(256), 0, s, S, P);
+        else hipLaunchKernelGGL((k_vol_occlude<false, false>), dim3(grid), dim3(256), 0, s, S, P);
     }
     vol_launch_check();
     if (stats) {
-        if (sph) hipLaunchKernelGGL((k_vol_shadow<true, true>), dim3(grid), dim3(256), 0, s, S, P, cur);
-        else hipLaunchKernelGGL((k_vol_shadow<true, false>), dim3(grid), dim3(256), 0, s, S, P, cur);
+        if (sph) hipLaunchKernelGGL((k_vol_shadow<true, true>), dim3(grid), dim3(256), 0, s, S, P);
+        else hipLaunchKernelGGL((k_vol_shadow<true, false>), dim3(grid), dim3(256), 0, s, S, P);
     } else {
-        if (sph) hipLaunchKernelGGL((k_vol_shadow<false, true>), dim3(grid), dim3(256), 0, s, S, P, cur);
-        else hipLaunchKernelGGL((k_vol_shadow<false, false>), dim3(grid), dim3(256), 0, s, S, P, cur);
+        if (sph) hipLaunchKernelGGL((k_vol_shadow<false, true>), dim3(grid), dim3(256), 0, s, S, P);
+        else hipLaunchKernelGGL((k_vol_shadow<false, false>), dim3(grid), dim3(256), 0, s, S, P);
     }
     vol_launch_check();
 }
