@@ -596,7 +596,7 @@ __device__ __forceinline__ void shade_surface(const DeviceScene &S, const PathBu
     if (b == 0) {
         // path_tracing.h:58-61
         if (v.area_light_id >= 0)
-            rad = rad + tp * light_emission(S, S.lights[v.area_light_id], -dir, LightPoint{v.pos, v.g.ng});
+            rad = rad + tp * light_emission(S.lights[v.area_light_id], -dir, LightPoint{v.pos, v.g.ng});
     } else {
         // path_tracing.h:243-322 for the vertex reached by the previous sample
         float4 pv = P.prev[pid];
@@ -607,9 +607,9 @@ __device__ __forceinline__ void shade_surface(const DeviceScene &S, const PathBu
         if (v.area_light_id >= 0) {
             const LightRec &l = S.lights[v.area_light_id];
             LightPoint lp{v.pos, v.g.ng};
-            D3 L = light_emission(S, l, -dir, lp);
+            D3 L = light_emission(l, -dir, lp);
             D3 C2 = G * f * L;
-            double p1 = S.light_pmf[v.area_light_id] * pdf_light_point(S, l, lp, org);
+            double p1 = S.light_pmf[v.area_light_id] * pdf_shape<SPH>(S.shapes[l.shape_id], lp, org);
             double w2 = (p2 * p2) / (p1 * p1 + p2 * p2);
             C2 = C2 / p2;
             rad = rad + tp * C2 * w2;
@@ -639,12 +639,12 @@ __device__ __forceinline__ void shade_surface(const DeviceScene &S, const PathBu
         D3 dir_light, L;
         double G = 0, tfar, lpdf;
         if (l.type == 0) {
-            LightPoint lp = sample_shape(S, S.shapes[l.shape_id], v.pos, lu0, lu1, sw);
+            LightPoint lp = sample_shape<SPH>(S, S.shapes[l.shape_id], v.pos, lu0, lu1, sw);
             dir_light = normalize(lp.pos - v.pos);
             double dl = sqrt(dist2(lp.pos, v.pos));
             tfar = (1 - S.eps) * dl;
             G = fmax(-dot(dir_light, lp.n), 0.0) / dist2(lp.pos, v.pos);
-            lpdf = pdf_shape(S.shapes[l.shape_id], lp, v.pos);
+            lpdf = pdf_shape<SPH>(S.shapes[l.shape_id], lp, v.pos);
             L = dot(lp.n, -dir_light) > 0 ? l.intensity : D3{0, 0, 0};
         } else {
             env_nee(l, lu0, lu1, dir_light, lpdf, L);
@@ -743,19 +743,18 @@ __device__ __forceinline__ void shade_queue(const DeviceScene &S, const PathBufs
 
 // The shading kernel of one material type (or, MT = -1, of the runtime-dispatch
 // bucket).  Occupancy of these FP64-heavy kernels is set by their register
-// count: the 2-wave variant caps it at 256 registers for the material types
-// whose code fits there with little or no spilling (Lambertian, RoughPlastic,
-// DisneyDiffuse, DisneyMetal, DisneySheen) and for DisneyBSDF, which spills
-// there but, running beside the other types' kernels, is faster at two waves
-// per SIMD than at one (shading of the 1080p large-mesh render 42.1 -> 40.6
-// ms); the others run one wave per SIMD.
+// count: 185-204 for Lambertian, RoughPlastic, DisneyDiffuse, DisneyMetal and
+// DisneySheen without spheres in the scene, under 257 with them, hence two
+// waves per SIMD; DisneyBSDF spills at two, but running beside the other
+// types' kernels is faster there than at one (shading of the 1080p large-mesh
+// render 42.1 -> 40.6 ms).  Three waves, which the first five reach with
+// little spilling, are slower, 43.0 against 35.4 ms for the same shading: the
+// kernels keep the vector-memory data unit 0.9 busy, and more waves beside
+// DisneyBSDF's only take its share of it.
+constexpr int shade_waves(int mt) { return mt == 2 || mt == 5 || mt == 6 || mt < 0 ? 1 : 2; }
 template <int MT, bool SPH, bool GUIDE>
-__global__ __launch_bounds__(256) void k_shade(DeviceScene S, PathBufs P, int cur) {
-    shade_queue<MT, SPH, GUIDE>(S, P, cur);
-}
-template <int MT, bool SPH, bool GUIDE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_shade_w2(DeviceScene S, PathBufs P,
-                                                                                         int cur) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(shade_waves(MT)))) void k_shade(
+    DeviceScene S, PathBufs P, int cur) {
     shade_queue<MT, SPH, GUIDE>(S, P, cur);
 }
 

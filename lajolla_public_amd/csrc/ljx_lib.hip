@@ -1093,15 +1093,15 @@ void shade_all_t(Scene &sc, PathBufs &P, int cur, int grid, int block, hipStream
     int next = 0;
     auto on = [&]() { return st[next++ % 3]; };
     // the heaviest kernels first, one per stream
-    if (m & (1u << 1)) launch(k_shade_w2<1, SPH, GUIDE>, grid, block, on(), S, P, cur);
-    if (m & (1u << 8)) launch(k_shade_w2<8, SPH, GUIDE>, grid, block, on(), S, P, cur);
-    if (m & (1u << 0)) launch(k_shade_w2<0, SPH, GUIDE>, grid, block, on(), S, P, cur);
+    if (m & (1u << 1)) launch(k_shade<1, SPH, GUIDE>, grid, block, on(), S, P, cur);
+    if (m & (1u << 8)) launch(k_shade<8, SPH, GUIDE>, grid, block, on(), S, P, cur);
+    if (m & (1u << 0)) launch(k_shade<0, SPH, GUIDE>, grid, block, on(), S, P, cur);
     if (m & (1u << 2)) launch(k_shade<2, SPH, GUIDE>, grid, block, on(), S, P, cur);
-    if (m & (1u << 3)) launch(k_shade_w2<3, SPH, GUIDE>, grid, block, on(), S, P, cur);
-    if (m & (1u << 4)) launch(k_shade_w2<4, SPH, GUIDE>, grid, block, on(), S, P, cur);
+    if (m & (1u << 3)) launch(k_shade<3, SPH, GUIDE>, grid, block, on(), S, P, cur);
+    if (m & (1u << 4)) launch(k_shade<4, SPH, GUIDE>, grid, block, on(), S, P, cur);
     if (m & (1u << 5)) launch(k_shade<5, SPH, GUIDE>, grid, block, on(), S, P, cur);
     if (m & (1u << 6)) launch(k_shade<6, SPH, GUIDE>, grid, block, on(), S, P, cur);
-    if (m & (1u << 7)) launch(k_shade_w2<7, SPH, GUIDE>, grid, block, on(), S, P, cur);
+    if (m & (1u << 7)) launch(k_shade<7, SPH, GUIDE>, grid, block, on(), S, P, cur);
     // unsorted bounces and textured materials go to the runtime-dispatch kernel
     if (P.sort_threshold > 0 || sc.has_textured) launch(k_shade<-1, SPH, GUIDE>, grid, block, on(), S, P, cur);
     launch(k_miss, grid, block, on(), S, P);

@@ -173,16 +173,18 @@ struct LightPoint {
 
 // sample_point_on_shape for triangle meshes and spheres
 // (src/shapes/triangle_mesh.inl:24-58, src/shapes/sphere.inl:164-212).
+// SPH: the scene has spheres.
+template <bool SPH>
 __device__ __forceinline__ LightPoint sample_shape(const DeviceScene &S, const ShapeRec &sh, D3 ref, double u0,
                                                   double u1, double w) {
-    if (sh.type == 0) {
+    if (SPH && sh.type == 0) {
         D3 c{sh.center[0], sh.center[1], sh.center[2]};
         double r = sh.radius;
         double s, co;
         if (dist2(ref, c) < r * r) {
             double z = 1 - 2 * u0;
             double r_ = sqrt(fmax(0.0, 1 - z * z));
-            sincos(2 * kPi * u1, &s, &co);
+            sincos_pi(2 * u1, s, co);
             D3 off{r_ * co, r_ * s, z};
             return {c + r * off, off};
         }
@@ -196,7 +198,7 @@ __device__ __forceinline__ LightPoint sample_shape(const DeviceScene &S, const S
         double ds = dc * ce - sqrt(fmax(0.0, r * r - dc * dc * se * se));
         double ca = (dc * dc + r * r - ds * ds) / (2 * dc * r);
         double sa = sqrt(fmax(0.0, 1 - ca * ca));
-        sincos(u1 * 2 * kPi, &s, &co);
+        sincos_pi(2 * u1, s, co);
         D3 n = -to_world(f, D3{sa * co, sa * s, ca});
         return {r * n + c, n};
     }
@@ -220,8 +222,9 @@ __device__ __forceinline__ LightPoint sample_shape(const DeviceScene &S, const S
     return {v0 + e1 * b1 + e2 * b2, ng};
 }
 // pdf_point_on_shape (src/shapes/triangle_mesh.inl:54-58, sphere.inl:218-238)
+template <bool SPH>
 __device__ __forceinline__ double pdf_shape(const ShapeRec &sh, const LightPoint &lp, D3 ref) {
-    if (sh.type == 0) {
+    if (SPH && sh.type == 0) {
         D3 c{sh.center[0], sh.center[1], sh.center[2]};
         double r = sh.radius;
         if (dist2(ref, c) < r * r) return 1 / (4 * kPi * r * r);
@@ -257,37 +260,6 @@ __device__ __forceinline__ void env_uv(D3 ld, double &u, double &v) {
     v = acos(clampd(ld.y, -1, 1)) * (1 / kPi);
     if (u < 0) u += 1;
 }
-// src/lights/envmap.inl:7-42
-__device__ __forceinline__ LightPoint sample_env(const LightRec &l, double u0, double u1) {
-    double eu, ev;
-    sample_env_uv(l, u0, u1, eu, ev);
-    double az = eu * (2 * kPi), el = ev * kPi;
-    double sa, ca, se, ce;
-    sincos(az, &sa, &ca);
-    sincos(el, &se, &ce);
-    D3 ld{sa * se, ce, -ca * se};
-    D3 wd = xform3(l.to_world, ld);
-    return {{0, 0, 0}, -wd};
-}
-__device__ __forceinline__ double pdf_env(const LightRec &l, D3 world_dir) {
-    D3 ld = xform3(l.to_local, world_dir);
-    double u, v;
-    env_uv(ld, u, v);
-    double ce = ld.y;
-    double se = sqrt(clampd(1 - ce * ce, 0, 1));
-    if (se <= 0) return 0;
-    return pdf_env_uv(l, u, v) / (2 * kPi * kPi * se);
-}
-__device__ __forceinline__ LightPoint sample_light_point(const DeviceScene &S, const LightRec &l, D3 ref, double u0,
-                                                        double u1, double w) {
-    if (l.type == 1) return sample_env(l, u0, u1);
-    return sample_shape(S, S.shapes[l.shape_id], ref, u0, u1, w);
-}
-__device__ __forceinline__ double pdf_light_point(const DeviceScene &S, const LightRec &l, const LightPoint &lp,
-                                                 D3 ref) {
-    if (l.type == 1) return pdf_env(l, -lp.n);
-    return pdf_shape(S.shapes[l.shape_id], lp, ref);
-}
 // Level-0 bilinear radiance of the envmap at lat-long (u, v) (src/mipmap.h:50-72; its
 // texels are the envmap's FP32 values).
 __device__ __forceinline__ D3 env_texel_bilinear(const LightRec &l, double u, double v) {
@@ -311,25 +283,19 @@ __device__ __forceinline__ void env_nee(const LightRec &l, double u0, double u1,
     double eu, ev;
     sample_env_uv(l, u0, u1, eu, ev);
     double sa, ca, se, ce;
-    sincos(eu * (2 * kPi), &sa, &ca);
-    sincos(ev * kPi, &se, &ce);
+    sincos_pi(2 * eu, sa, ca);
+    sincos_pi(ev, se, ce);
     dir = xform3(l.to_world, D3{sa * se, ce, -ca * se});
     pdf = se > 0 ? pdf_env_uv(l, eu, ev) / (2 * kPi * kPi * se) : 0.0;
     L = env_texel_bilinear(l, eu, ev) * l.scale;
 }
 
-// emission (src/lights/diffuse_area_light.inl:15-20; src/lights/envmap.inl:44-72).
-// The envmap's footprint, min(|du/dw|, dv/dw), is never positive (dv/dw < 0),
-// so the reference reads the image bilinearly on level 0; only along the exact
+// Emission of an area light (src/lights/diffuse_area_light.inl:15-20), the
+// only kind a ray can hit; escaped rays read the envmap in k_miss.  The
+// envmap's footprint, min(|du/dw|, dv/dw), is never positive (dv/dw < 0), so
+// the reference reads the image bilinearly on level 0; only along the exact
 // poles, where that footprint is NaN, would it read the last level instead.
-__device__ __forceinline__ D3 light_emission(const DeviceScene &S, const LightRec &l, D3 view_dir,
-                                            const LightPoint &lp) {
-    if (l.type == 1) {
-        D3 w = xform3(l.to_local, -view_dir);
-        double u, v;
-        env_uv(w, u, v);
-        return env_texel_bilinear(l, u, v) * l.scale;
-    }
+__device__ __forceinline__ D3 light_emission(const LightRec &l, D3 view_dir, const LightPoint &lp) {
     if (dot(lp.n, view_dir) <= 0) return {0, 0, 0};
     return l.intensity;
 }

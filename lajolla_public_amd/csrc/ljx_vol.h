@@ -287,13 +287,13 @@ __device__ __forceinline__ void vol_shade(const DeviceScene &S, const PathBufs &
         if (v.area_light_id >= 0) {
             const LightRec &l = S.lights[v.area_light_id];
             LightPoint lp{v.pos, v.g.ng};
-            D3 add = tp * light_emission(S, l, -dir, lp);
+            D3 add = tp * light_emission(l, -dir, lp);
             const float4 mt = P.mtp[pid];
             if (mt.w == 0.f) {  // some vertex of the path scattered
                 const float4 nc = P.nee_c[pid];
                 const D3 nee_p_cache{nc.x, nc.y, nc.z};
                 const D3 multi_trans_pdf = D3{mt.x, mt.y, mt.z} * trans_dir_pdf;
-                double pdf_nee = S.light_pmf[v.area_light_id] * pdf_light_point(S, l, lp, nee_p_cache);
+                double pdf_nee = S.light_pmf[v.area_light_id] * pdf_shape<SPH>(S.shapes[l.shape_id], lp, nee_p_cache);
                 double G = fabs(dot(dir, v.g.ng)) / dist2(nee_p_cache, v.pos);
                 double dp = double(nc.w) * avgc(multi_trans_pdf) * G;
                 add = add * ((dp * dp) / (dp * dp + pdf_nee * pdf_nee));
@@ -331,10 +331,10 @@ __device__ __forceinline__ void vol_shade(const DeviceScene &S, const PathBufs &
         if (S.num_lights > 0) {
             int lid = sample_cdf_guided(S.light_cdf, S.num_lights, lw, S.light_guide, S.light_guide_m);
             const LightRec &l = S.lights[lid];
-            LightPoint lp = sample_light_point(S, l, pos, lu0, lu1, sw);
+            LightPoint lp = sample_shape<SPH>(S, S.shapes[l.shape_id], pos, lu0, lu1, sw);
             D3 dir_light = normalize(lp.pos - pos);
             double G = fmax(-dot(dir_light, lp.n), 0.0) / dist2(pos, lp.pos);
-            double pdf_nee = S.light_pmf[lid] * pdf_light_point(S, l, lp, pos);
+            double pdf_nee = S.light_pmf[lid] * pdf_shape<SPH>(S.shapes[l.shape_id], lp, pos);
             if (G > 0 && pdf_nee > 0) {
                 D3 f;
                 double pdf_f;
@@ -350,7 +350,7 @@ __device__ __forceinline__ void vol_shade(const DeviceScene &S, const PathBufs &
                     f = bsdf_eval<DMT>(mat, dir_view, dir_light, v.g);
                     pdf_f = bsdf_pdf<DMT>(mat, dir_view, dir_light, v.g);
                 }
-                D3 L = light_emission(S, l, -dir_light, lp);
+                D3 L = light_emission(l, -dir_light, lp);
                 D3 K = pre * G * f * L;
                 if (K.x != 0 || K.y != 0 || K.z != 0) {
                     push_sh = true;
