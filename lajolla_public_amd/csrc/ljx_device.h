@@ -868,17 +868,10 @@ LJX_HD BsdfSample disney_bsdf_sample(const MatRec &m, D3 in, const ShadeGeom &g,
 // MT is the material type tag of include/lajolla_amd.h; MT = -1 dispatches
 // at run time.  Shading kernels are instantiated per type so that each
 // sorted bucket runs straight-line code.
-// The material type a BSDF call switches on: MT itself in a kernel of one
-// type; the record's own type under runtime dispatch (MT = -1); and under
-// runtime dispatch over lajolla's three basic materials only (MT =
-// kMtBasic: Lambertian, RoughPlastic, RoughDielectric; the host picks it
-// only for scenes that use no other type) the type clamped to them, so the
-// Disney lobes drop out of the kernel and its register budget.
-constexpr int kMtBasic = -2;
+// The material type a BSDF call switches on.
 template <int MT>
 LJX_HD int dispatch_type(const MatRec &m) {
     if constexpr (MT >= 0) return MT;
-    else if constexpr (MT == kMtBasic) return m.type < 2 ? m.type : 2;
     else return m.type;
 }
 

@@ -751,9 +751,11 @@ __device__ __forceinline__ void shade_queue(const DeviceScene &S, const PathBufs
 // little spilling, are slower, 43.0 against 35.4 ms for the same shading: the
 // kernels keep the vector-memory data unit 0.9 busy, and more waves beside
 // DisneyBSDF's only take its share of it.
-constexpr int shade_waves(int mt) { return mt == 2 || mt == 5 || mt == 6 || mt < 0 ? 1 : 2; }
+// RoughDielectric, DisneyGlass and DisneyClearcoat need four registers more
+// than two waves allow without spheres, and too many with them.
+constexpr int shade_waves(int mt, bool sph) { return mt < 0 || (sph && (mt == 2 || mt == 5 || mt == 6)) ? 1 : 2; }
 template <int MT, bool SPH, bool GUIDE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(shade_waves(MT)))) void k_shade(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(shade_waves(MT, SPH)))) void k_shade(
     DeviceScene S, PathBufs P, int cur) {
     shade_queue<MT, SPH, GUIDE>(S, P, cur);
 }

@@ -1157,7 +1157,7 @@ void vol_stage(Scene &sc, PathBufs &P, int n, int cur, int grid, hipStream_t s, 
     sort_ext_queue(P, n, cur, s);
     hipStream_t st[3];
     fan_out(sc, s, fan, st);
-    vol_shade_all(sc.ds, P, cur, grid, st, sc.has_spheres, (sc.mat_types_present & ~7u) == 0);
+    vol_shade_all(sc.ds, P, cur, grid, st, sc.has_spheres, sc.mat_types_present, sc.has_textured);
     fan_in(sc, s, fan);
 }
 

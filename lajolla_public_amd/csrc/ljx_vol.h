@@ -317,6 +317,14 @@ __device__ __forceinline__ void vol_shade(const DeviceScene &S, const PathBufs &
         push_ext = true;
         return;
     } else {
+        // constant materials are read in place; the runtime-dispatch kernel, which
+        // also takes textured ones, works on a copy with the textures evaluated
+        MatRec mat_tex;
+        if constexpr (EV == kEvSurface && DMT < 0) {
+            mat_tex = S.materials[v.material_id];
+            if (mat_tex.textured) resolve_textures(S, mat_tex, v.tu, v.tv, 0.0);
+        }
+        const MatRec &mat = DMT < 0 ? mat_tex : S.materials[scatter ? 0 : v.material_id];
         D3 dir_view = -dir;
         // NEE sub-stream
         uint32_t k = pcg_next(st, inc);
@@ -345,8 +353,6 @@ __device__ __forceinline__ void vol_shade(const DeviceScene &S, const PathBufs &
                     pdf_f = pv;
                     pre = pre * sigma_s;
                 } else {
-                    MatRec mat = S.materials[v.material_id];
-                    if (mat.textured) resolve_textures(S, mat, v.tu, v.tv, 0.0);
                     f = bsdf_eval<DMT>(mat, dir_view, dir_light, v.g);
                     pdf_f = bsdf_pdf<DMT>(mat, dir_view, dir_light, v.g);
                 }
@@ -374,8 +380,6 @@ __device__ __forceinline__ void vol_shade(const DeviceScene &S, const PathBufs &
             tp = tp * (D3{dir_pdf, dir_pdf, dir_pdf} / dir_pdf) * sigma_s;
             tnear = 0.f;
         } else {
-            MatRec mat = S.materials[v.material_id];
-            if (mat.textured) resolve_textures(S, mat, v.tu, v.tv, 0.0);
             double u0 = pcg_double(st, inc), u1 = pcg_double(st, inc), w = pcg_double(st, inc);
             BsdfSample bs = bsdf_sample<DMT>(mat, dir_view, v.g, u0, u1, w);
             if (!bs.valid) return;
@@ -406,11 +410,13 @@ __device__ __forceinline__ void vol_shade(const DeviceScene &S, const PathBufs &
     }
 }
 
+// Surfaces: DMT is the material type of the kernel's bucket, or -1 for the
+// buckets from kVolTyped on.
+constexpr int kVolTyped = 3;
 template <bool SPH, int DMT, int EV>
-__global__ __launch_bounds__(256) void k_vol_shade(DeviceScene S, PathBufs P, int cur) {
-    // surface buckets of all material types lie together
-    constexpr int first = EV == kEvScatter ? kBucketScatter : EV == kEvSurface ? 0 : kBucketNoMat;
-    constexpr int end = EV == kEvSurface ? kBucketScatter : first + 1;
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EV == kEvSurface && DMT >= 0 && !SPH ? 2 : 1))) void k_vol_shade(DeviceScene S, PathBufs P, int cur) {
+    constexpr int first = EV == kEvScatter ? kBucketScatter : EV == kEvPass ? kBucketNoMat : DMT >= 0 ? DMT : kVolTyped;
+    constexpr int end = EV == kEvSurface && DMT < 0 ? kBucketScatter : first + 1;
     const int j0 = bucket_start(P, first), j1 = bucket_start(P, end);
     for (int j = j0 + blockIdx.x * blockDim.x + threadIdx.x; j < j1; j += gridDim.x * blockDim.x) {
         const uint32_t pid = P.order[j];
@@ -713,20 +719,24 @@ inline void vol_events(const DeviceScene &S, PathBufs &P, int cur, int grid, hip
     vol_launch_check();
 }
 // The shading kernels, on the streams given (one may stand for all three).
-// basic: the scene uses no material types beyond lajolla's three basic ones.
+// types: the material types present; textured: some material reads a texture.
 template <bool SPH>
-void vol_shade_t(const DeviceScene &S, PathBufs &P, int cur, int grid, const hipStream_t (&s)[3], bool basic) {
+void vol_shade_t(const DeviceScene &S, PathBufs &P, int cur, int grid, const hipStream_t (&s)[3], unsigned types,
+                 bool textured) {
     const dim3 g(grid), b(256);
-    if (basic) hipLaunchKernelGGL((k_vol_shade<SPH, kMtBasic, kEvSurface>), g, b, 0, s[0], S, P, cur);
-    else hipLaunchKernelGGL((k_vol_shade<SPH, -1, kEvSurface>), g, b, 0, s[0], S, P, cur);
-    hipLaunchKernelGGL((k_vol_shade<SPH, kMtBasic, kEvScatter>), g, b, 0, s[1], S, P, cur);
-    hipLaunchKernelGGL((k_vol_shade<SPH, kMtBasic, kEvPass>), g, b, 0, s[2], S, P, cur);
+    if (types & 4) hipLaunchKernelGGL((k_vol_shade<SPH, 2, kEvSurface>), g, b, 0, s[0], S, P, cur);
+    hipLaunchKernelGGL((k_vol_shade<SPH, 0, kEvScatter>), g, b, 0, s[1], S, P, cur);
+    if (types & 1) hipLaunchKernelGGL((k_vol_shade<SPH, 0, kEvSurface>), g, b, 0, s[2], S, P, cur);
+    if (types & 2) hipLaunchKernelGGL((k_vol_shade<SPH, 1, kEvSurface>), g, b, 0, s[0], S, P, cur);
+    if (textured || (types >> kVolTyped))
+        hipLaunchKernelGGL((k_vol_shade<SPH, -1, kEvSurface>), g, b, 0, s[0], S, P, cur);
+    hipLaunchKernelGGL((k_vol_shade<SPH, 0, kEvPass>), g, b, 0, s[2], S, P, cur);
     vol_launch_check();
 }
 inline void vol_shade_all(const DeviceScene &S, PathBufs &P, int cur, int grid, const hipStream_t (&s)[3], bool sph,
-                          bool basic) {
-    if (sph) vol_shade_t<true>(S, P, cur, grid, s, basic);
-    else vol_shade_t<false>(S, P, cur, grid, s, basic);
+                          unsigned types, bool textured) {
+    if (sph) vol_shade_t<true>(S, P, cur, grid, s, types, textured);
+    else vol_shade_t<false>(S, P, cur, grid, s, types, textured);
 }
 
 inline void vol_shadow(const DeviceScene &S, PathBufs &P, int grid, hipStream_t s, bool stats, bool sph) {
