@@ -962,6 +962,27 @@ LJX_HD D3 vol_lookup(const VolumeRec &v, D3 p) {
     return v.scale * acc;
 }
 
+// The same for a volume of one channel.
+LJX_HD double vol_lookup_grey(const VolumeRec &v, D3 p) {
+    if (v.type == 0) return v.scale * v.value.x;
+    D3 pn = (p - v.p_min) / (v.p_max - v.p_min);
+    if (pn.x < 0 || pn.x > 1 || pn.y < 0 || pn.y > 1 || pn.z < 0 || pn.z > 1) return 0;
+    pn.x *= double(v.rx - 1);
+    pn.y *= double(v.ry - 1);
+    pn.z *= double(v.rz - 1);
+    const int x0 = min(max(int(pn.x), 0), v.rx - 1), x1 = min(x0 + 1, v.rx - 1);
+    const int y0 = min(max(int(pn.y), 0), v.ry - 1), y1 = min(y0 + 1, v.ry - 1);
+    const int z0 = min(max(int(pn.z), 0), v.rz - 1), z1 = min(z0 + 1, v.rz - 1);
+    const double dx = pn.x - x0, dy = pn.y - y0, dz = pn.z - z0;
+    const float *r00 = v.data + (size_t(z0) * v.ry + y0) * v.rx, *r10 = v.data + (size_t(z0) * v.ry + y1) * v.rx;
+    const float *r01 = v.data + (size_t(z1) * v.ry + y0) * v.rx, *r11 = v.data + (size_t(z1) * v.ry + y1) * v.rx;
+    const double acc = r00[x0] * ((1 - dx) * (1 - dy) * (1 - dz)) + r00[x1] * (dx * (1 - dy) * (1 - dz)) +
+                       r10[x0] * ((1 - dx) * dy * (1 - dz)) + r10[x1] * (dx * dy * (1 - dz)) +
+                       r01[x0] * ((1 - dx) * (1 - dy) * dz) + r01[x1] * (dx * (1 - dy) * dz) +
+                       r11[x0] * ((1 - dx) * dy * dz) + r11[x1] * (dx * dy * dz);
+    return v.scale * acc;
+}
+
 // src/volume.h:120-144: does the ray's [0, tfar] reach the grid box (pbrt's slab test)
 LJX_HD bool vol_hit(const VolumeRec &v, D3 o, D3 d, double tfar) {
     if (v.type == 0) return true;

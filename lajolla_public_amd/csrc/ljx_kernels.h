@@ -99,6 +99,7 @@ struct PathBufs {
     int spp, max_depth, rr_depth;
     int volpath;
     int vol_flight;  // free flight runs in k_vol_flight (scenes with grid media), else inside k_vol_shade
+    int vol_grey;    // every medium is a grid of one density channel
     int max_null;
     uint64_t seed;
     // learned guiding (path integrator)

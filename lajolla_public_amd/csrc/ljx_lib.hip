@@ -206,6 +206,7 @@ struct Scene {
     bool has_textured = false;  // some material reads a texture: shaded by the runtime-dispatch kernel
     bool has_media = false;
     bool has_grid_media = false;  // a heterogeneous medium: long delta-tracking loops
+    bool grey_media = false;      // all are, each with one density channel (or a grey constant)
     int num_media = 0;
     double bound_center[3] = {0, 0, 0};
     double bound_radius = 0;
@@ -790,6 +791,12 @@ void build_scene(Scene &sc, const ljx_scene_desc *d) {
         }
     }
 
+    sc.grey_media = sc.has_grid_media;
+    for (const MediumRec &m : media)
+        sc.grey_media = sc.grey_media && m.type != 0 &&
+                        (m.density.type == 0 ? m.density.value.x == m.density.value.y && m.density.value.x == m.density.value.z
+                                             : m.density.channels == 1);
+
     // ---- camera (src/camera.cpp:7-21)
     S.camera = make_camera(d->camera);
 
@@ -1299,6 +1306,7 @@ void render_impl(Scene &sc, const ljx_render_options *o, const ljx_exec_options 
     P.seed = opt.seed;
     P.volpath = vol ? 1 : 0;
     P.vol_flight = vol && sc.has_grid_media ? 1 : 0;
+    P.vol_grey = vol && sc.grey_media ? 1 : 0;
     P.max_null = opt.max_null_collisions;
     P.rec_depth = 0;
     P.jobs = nullptr;
@@ -1679,6 +1687,7 @@ void batch_impl(const ljx_batch_job *jobs, size_t njobs, const ljx_exec_options 
             P.seed = 0;
             P.volpath = vol ? 1 : 0;
             P.vol_flight = vol && sc.has_grid_media ? 1 : 0;
+            P.vol_grey = vol && sc.grey_media ? 1 : 0;
             P.max_null = sc.options.max_null_collisions;
             P.rec_depth = 0;
             P.jobs = gp.dtable;
