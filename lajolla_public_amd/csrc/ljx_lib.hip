@@ -559,24 +559,24 @@ void build_scene(Scene &sc, const ljx_scene_desc *d) {
             r.has_uvs = s.uvs != nullptr;
             r.tri_offset = int(tri_vidx.size() / 3);
             r.num_tris = int(s.num_triangles);
-            for (uint64_t v = 0; v < s.num_vertices; v++) {
+            // whole arrays at a time: a push_back per value took 5 ms longer for 2.3M triangles
+            const size_t nv = size_t(s.num_vertices), nt = size_t(s.num_triangles);
+            vpos.insert(vpos.end(), s.positions, s.positions + 3 * nv);
+            for (size_t v = 0; v < nv; v++)
                 for (int k = 0; k < 3; k++) {
-                    float p = s.positions[3 * v + k];
-                    vpos.push_back(p);
-                    lo[k] = std::min(lo[k], p);
-                    hi[k] = std::max(hi[k], p);
-                    vnrm.push_back(s.normals ? s.normals[3 * v + k] : 0.f);
+                    lo[k] = std::min(lo[k], s.positions[3 * v + k]);
+                    hi[k] = std::max(hi[k], s.positions[3 * v + k]);
                 }
-                vuv.push_back(s.uvs ? s.uvs[2 * v] : 0.f);
-                vuv.push_back(s.uvs ? s.uvs[2 * v + 1] : 0.f);
-            }
-            for (uint64_t t = 0; t < s.num_triangles; t++) {
-                tri_vidx.push_back(s.indices[3 * t] + voff);
-                tri_vidx.push_back(s.indices[3 * t + 1] + voff);
-                tri_vidx.push_back(s.indices[3 * t + 2] + voff);
-                prim_shape.push_back(i);
-                prim_local.push_back(int(t));
-            }
+            if (s.normals) vnrm.insert(vnrm.end(), s.normals, s.normals + 3 * nv);
+            else vnrm.resize(vnrm.size() + 3 * nv);
+            if (s.uvs) vuv.insert(vuv.end(), s.uvs, s.uvs + 2 * nv);
+            else vuv.resize(vuv.size() + 2 * nv);
+            const size_t t0 = tri_vidx.size(), p0 = prim_local.size();
+            tri_vidx.resize(t0 + 3 * nt);
+            for (size_t t = 0; t < 3 * nt; t++) tri_vidx[t0 + t] = s.indices[t] + voff;
+            prim_shape.resize(p0 + nt, i);
+            prim_local.resize(p0 + nt);
+            for (size_t t = 0; t < nt; t++) prim_local[p0 + t] = int(t);
             // triangle areas in FP64 (src/shapes/triangle_mesh.inl:60-75): the
             // light's pdf and its triangle table, so emitting shapes only
             const bool emits = s.area_light_id >= 0 || light_shape[i];
