@@ -104,6 +104,17 @@ def test_single_triangle_and_one_wave_ranges():
         check_same(s, f"{n} triangles")
 
 
+@pytest.mark.parametrize("n", [127, 128, 129, 255, 257])
+def test_one_wave_range_limit(n):
+    """Around the largest range that one wave builds."""
+    rng = np.random.default_rng(n)
+    s = scenes.SceneDesc()
+    m = s.add_material(0, (0.5, 0.5, 0.5))
+    P = (rng.uniform(-5, 5, (n, 1, 3)) + rng.normal(scale=0.1, size=(n, 3, 3))).reshape(-1, 3).astype(np.float32)
+    s.add_mesh(P, np.arange(3 * n, dtype=np.int32).reshape(n, 3), m)
+    check_same(s, f"{n} triangles")
+
+
 def test_node_fetch_rate():
     """The random node-fetch rate: positive, higher with every lane of a
     wave fetching than with eight, and argument errors cross the boundary."""
