@@ -40,10 +40,11 @@ namespace {
 constexpr int kChunk = 2048;  // primitives per block in the wide-range kernels
 // Ranges of at most this many primitives are built by one wave.  At 512 a
 // wave's boxes and bins take 19 KB of LDS, two waves per SIMD, and a wave
-// hides nothing of its serial steps; at 128 it is 6.7 KB and six waves: the
-// narrow ranges of 2.3M triangles 11.5 -> 8.1 ms, for 1.4 ms more of wide
-// levels (256: 8.9 and 0.5; 64: 7.7 and 3.1).
-constexpr int kSmall = 128;
+// hides nothing of its serial steps; at 256 it is 11 KB and three to four: the
+// narrow ranges of 2.3M triangles 11.5 -> 8.9 ms for 0.5 ms more of wide
+// levels, opening the scene 43.5 -> 41.1 ms.  At 128 the wide levels grow by
+// 1.4 ms and their bins to 48 MB: 42.1 ms.
+constexpr int kSmall = 256;
 constexpr int kWaveStack = 32;
 constexpr int kBinInts = 3 * kBvhBins * 7;  // per bin: count, lo xyz, hi xyz
 
