@@ -14,7 +14,7 @@
 //    split (one lane per range), then a stable partition by per-chunk counts,
 //    their scan per range and a block-level scan of the flags;
 //  * narrow ranges are built to their leaves by one wave each: bounds by wave
-//    reduction, bins in LDS, the split by three lanes (one per axis), a
+//    reduction, bins in LDS, the split by the wave (a lane per bin), a
 //    ballot-ranked stable partition staged through LDS, and a stack of
 //    pending ranges (the larger pushed, the smaller taken next, so it stays
 //    logarithmic);
