@@ -868,6 +868,9 @@ LJX_HD BsdfSample disney_bsdf_sample(const MatRec &m, D3 in, const ShadeGeom &g,
 // MT is the material type tag of include/lajolla_amd.h; MT = -1 dispatches
 // at run time.  Shading kernels are instantiated per type so that each
 // sorted bucket runs straight-line code.
+// MT = kMtEnv: run-time dispatch in a kernel whose lights may be envmaps
+// where the others take area lights only (light_emission).
+constexpr int kMtEnv = -2;
 // The material type a BSDF call switches on.
 template <int MT>
 LJX_HD int dispatch_type(const MatRec &m) {

@@ -597,7 +597,7 @@ __device__ __forceinline__ void shade_surface(const DeviceScene &S, const PathBu
     if (b == 0) {
         // path_tracing.h:58-61
         if (v.area_light_id >= 0)
-            rad = rad + tp * light_emission(S.lights[v.area_light_id], -dir, LightPoint{v.pos, v.g.ng});
+            rad = rad + tp * light_emission<MT == kMtEnv>(S.lights[v.area_light_id], -dir, LightPoint{v.pos, v.g.ng});
     } else {
         // path_tracing.h:243-322 for the vertex reached by the previous sample
         float4 pv = P.prev[pid];
@@ -608,9 +608,9 @@ __device__ __forceinline__ void shade_surface(const DeviceScene &S, const PathBu
         if (v.area_light_id >= 0) {
             const LightRec &l = S.lights[v.area_light_id];
             LightPoint lp{v.pos, v.g.ng};
-            D3 L = light_emission(l, -dir, lp);
+            D3 L = light_emission<MT == kMtEnv>(l, -dir, lp);
             D3 C2 = G * f * L;
-            double p1 = S.light_pmf[v.area_light_id] * pdf_shape<SPH>(S.shapes[l.shape_id], lp, org);
+            double p1 = S.light_pmf[v.area_light_id] * pdf_light_point<SPH, MT == kMtEnv>(S, l, lp, org);
             double w2 = (p2 * p2) / (p1 * p1 + p2 * p2);
             C2 = C2 / p2;
             rad = rad + tp * C2 * w2;
@@ -718,11 +718,13 @@ __device__ __forceinline__ void shade_surface(const DeviceScene &S, const PathBu
     P.rad[pid] = make_float4(float(rad.x), float(rad.y), float(rad.z), 0.f);
 }
 
-// MT = -1: the unsorted bucket, with the material type dispatched per path.
+// MT = -1: the unsorted bucket, with the material type dispatched per path;
+// kMtEnv: so for every bucket of hits.
 template <int MT, bool SPH, bool GUIDE>
 __device__ __forceinline__ void shade_queue(const DeviceScene &S, const PathBufs &P, int cur) {
-    constexpr int B = MT >= 0 ? MT : kBucketAny;
-    const int n = P.ctr[C_BUCKET + B], start = bucket_start(P, B);
+    constexpr int B = MT >= 0 ? MT : MT == kMtEnv ? 0 : kBucketAny;
+    const int start = bucket_start(P, B);
+    const int n = MT == kMtEnv ? bucket_start(P, kBucketAny + 1) : P.ctr[C_BUCKET + B];
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const int j = start + i;
         const uint32_t pid = P.order[j];
@@ -742,8 +744,7 @@ __device__ __forceinline__ void shade_queue(const DeviceScene &S, const PathBufs
     }
 }
 
-// The shading kernel of one material type (or, MT = -1, of the runtime-dispatch
-// bucket).  Occupancy of these FP64-heavy kernels is set by their register
+// The shading kernel of one material type (or, MT < 0, of run-time dispatch).  Occupancy of these FP64-heavy kernels is set by their register
 // count: 185-204 for Lambertian, RoughPlastic, DisneyDiffuse, DisneyMetal and
 // DisneySheen without spheres in the scene, under 257 with them, hence two
 // waves per SIMD; DisneyBSDF spills at two, but running beside the other

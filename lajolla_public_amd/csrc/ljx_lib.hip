@@ -204,6 +204,8 @@ struct Scene {
     bool has_spheres = false;
     unsigned mat_types_present = 0;
     bool has_textured = false;  // some material reads a texture: shaded by the runtime-dispatch kernel
+    bool env_lights = false;    // an envmap is among the lights
+    bool env_emitters = false;  // ... and some shape has it as its area light
     bool has_media = false;
     bool has_grid_media = false;  // a heterogeneous medium: long delta-tracking loops
     bool grey_media = false;      // all are, each with one density channel (or a grey constant)
@@ -745,6 +747,11 @@ void build_scene(Scene &sc, const ljx_scene_desc *d) {
             power[i] = luminance_h(l.intensity) * area * kPi;
         }
     }
+    for (int i = 0; i < d->num_lights; i++) sc.env_lights = sc.env_lights || d->lights[i].type == LJX_LIGHT_ENVMAP;
+    for (int i = 0; i < d->num_shapes; i++) {
+        const int lid = d->shapes[i].area_light_id;
+        sc.env_emitters = sc.env_emitters || (lid >= 0 && d->lights[lid].type == LJX_LIGHT_ENVMAP);
+    }
     std::vector<double> lpmf, lcdf;
     if (d->num_lights > 0) make_dist(power, lpmf, lcdf);
 
@@ -1099,6 +1106,13 @@ void shade_all_t(Scene &sc, PathBufs &P, int cur, int grid, int block, hipStream
     fan_out(sc, s, fan, st);
     int next = 0;
     auto on = [&]() { return st[next++ % 3]; };
+    if (sc.env_emitters) {
+        // one kernel shades every hit (the one for spheres takes scenes without them too)
+        launch(k_shade<kMtEnv, true, GUIDE>, grid, block, on(), S, P, cur);
+        launch(k_miss, grid, block, on(), S, P);
+        fan_in(sc, s, fan);
+        return;
+    }
     // the heaviest kernels first, one per stream
     if (m & (1u << 1)) launch(k_shade<1, SPH, GUIDE>, grid, block, on(), S, P, cur);
     if (m & (1u << 8)) launch(k_shade<8, SPH, GUIDE>, grid, block, on(), S, P, cur);
@@ -1164,7 +1178,7 @@ void vol_stage(Scene &sc, PathBufs &P, int n, int cur, int grid, hipStream_t s, 
     sort_ext_queue(P, n, cur, s);
     hipStream_t st[3];
     fan_out(sc, s, fan, st);
-    vol_shade_all(sc.ds, P, cur, grid, st, sc.has_spheres, sc.mat_types_present, sc.has_textured);
+    vol_shade_all(sc.ds, P, cur, grid, st, sc.has_spheres, sc.mat_types_present, sc.has_textured, sc.env_lights);
     fan_in(sc, s, fan);
 }
 

@@ -290,14 +290,60 @@ __device__ __forceinline__ void env_nee(const LightRec &l, double u0, double u1,
     L = env_texel_bilinear(l, eu, ev) * l.scale;
 }
 
-// Emission of an area light (src/lights/diffuse_area_light.inl:15-20), the
-// only kind a ray can hit; escaped rays read the envmap in k_miss.  The
-// envmap's footprint, min(|du/dw|, dv/dw), is never positive (dv/dw < 0), so
-// the reference reads the image bilinearly on level 0; only along the exact
+// A light at a point of it: emission, the point's sampling and its pdf.
+// Nearly every light that a ray hits or a volumetric path samples is an area
+// light, and the kernels of such scenes are compiled for those alone: an
+// envmap's l.shape_id names no shape.  A description may still give a shape an
+// envmap as its area light, or list an envmap that it does not name as the
+// scene's; the host launches the kernels with ENV (kMtEnv), which test the
+// type, for the scenes that hold such a light where the integrator meets it
+// (Scene::env_emitters, Scene::env_lights).
+// Emission (src/lights/diffuse_area_light.inl:15-20; src/lights/envmap.inl:44-72).
+// The envmap's footprint, min(|du/dw|, dv/dw), is never positive (dv/dw < 0),
+// so the reference reads the image bilinearly on level 0; only along the exact
 // poles, where that footprint is NaN, would it read the last level instead.
+template <bool ENV>
 __device__ __forceinline__ D3 light_emission(const LightRec &l, D3 view_dir, const LightPoint &lp) {
+    if constexpr (ENV) {
+        if (l.type == 1) {
+            double u, v;
+            env_uv(xform3(l.to_local, -view_dir), u, v);
+            return env_texel_bilinear(l, u, v) * l.scale;
+        }
+    }
     if (dot(lp.n, view_dir) <= 0) return {0, 0, 0};
     return l.intensity;
+}
+// src/lights/envmap.inl:7-20
+template <bool SPH, bool ENV>
+__device__ __forceinline__ LightPoint sample_light_point(const DeviceScene &S, const LightRec &l, D3 ref, double u0,
+                                                        double u1, double w) {
+    if constexpr (ENV) {
+        if (l.type == 1) {
+            double eu, ev;
+            sample_env_uv(l, u0, u1, eu, ev);
+            double sa, ca, se, ce;
+            sincos_pi(2 * eu, sa, ca);
+            sincos_pi(ev, se, ce);
+            return {{0, 0, 0}, -xform3(l.to_world, D3{sa * se, ce, -ca * se})};
+        }
+    }
+    return sample_shape<SPH>(S, S.shapes[l.shape_id], ref, u0, u1, w);
+}
+// src/lights/envmap.inl:22-42
+template <bool SPH, bool ENV>
+__device__ __forceinline__ double pdf_light_point(const DeviceScene &S, const LightRec &l, const LightPoint &lp,
+                                                 D3 ref) {
+    if constexpr (ENV) {
+        if (l.type == 1) {
+            const D3 ld = xform3(l.to_local, -lp.n);
+            double u, v;
+            env_uv(ld, u, v);
+            const double se = sqrt(clampd(1 - ld.y * ld.y, 0, 1));
+            return se > 0 ? pdf_env_uv(l, u, v) / (2 * kPi * kPi * se) : 0.0;
+        }
+    }
+    return pdf_shape<SPH>(S.shapes[l.shape_id], lp, ref);
 }
 
 }  // namespace ljx

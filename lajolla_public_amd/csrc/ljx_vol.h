@@ -277,7 +277,7 @@ constexpr int kEvScatter = 0, kEvSurface = 1, kEvPass = 2;
 template <bool SPH, int DMT, int EV>
 __device__ __forceinline__ void vol_shade(const DeviceScene &S, const PathBufs &P, uint32_t pid, bool &push_ext,
                                           bool &push_sh, float4 &sh_o, float4 &sh_d, float4 &sh_c, float4 &sh_x) {
-    constexpr bool scatter = EV == kEvScatter;
+    constexpr bool scatter = EV == kEvScatter, ENV = DMT == kMtEnv;
     push_ext = false;
     push_sh = false;
     float4 ro = P.ray_o[pid], rd = P.ray_d[pid];
@@ -323,13 +323,13 @@ __device__ __forceinline__ void vol_shade(const DeviceScene &S, const PathBufs &
         if (v.area_light_id >= 0) {
             const LightRec &l = S.lights[v.area_light_id];
             LightPoint lp{v.pos, v.g.ng};
-            D3 add = tp * light_emission(l, -dir, lp);
+            D3 add = tp * light_emission<ENV>(l, -dir, lp);
             const float4 mt = P.mtp[pid];
             if (mt.w == 0.f) {  // some vertex of the path scattered
                 const float4 nc = P.nee_c[pid];
                 const D3 nee_p_cache{nc.x, nc.y, nc.z};
                 const D3 multi_trans_pdf = D3{mt.x, mt.y, mt.z} * trans_dir_pdf;
-                double pdf_nee = S.light_pmf[v.area_light_id] * pdf_shape<SPH>(S.shapes[l.shape_id], lp, nee_p_cache);
+                double pdf_nee = S.light_pmf[v.area_light_id] * pdf_light_point<SPH, ENV>(S, l, lp, nee_p_cache);
                 double G = fabs(dot(dir, v.g.ng)) / dist2(nee_p_cache, v.pos);
                 double dp = double(nc.w) * avgc(multi_trans_pdf) * G;
                 add = add * ((dp * dp) / (dp * dp + pdf_nee * pdf_nee));
@@ -375,10 +375,10 @@ __device__ __forceinline__ void vol_shade(const DeviceScene &S, const PathBufs &
         if (S.num_lights > 0) {
             int lid = sample_cdf_guided(S.light_cdf, S.num_lights, lw, S.light_guide, S.light_guide_m);
             const LightRec &l = S.lights[lid];
-            LightPoint lp = sample_shape<SPH>(S, S.shapes[l.shape_id], pos, lu0, lu1, sw);
+            LightPoint lp = sample_light_point<SPH, ENV>(S, l, pos, lu0, lu1, sw);
             D3 dir_light = normalize(lp.pos - pos);
             double G = fmax(-dot(dir_light, lp.n), 0.0) / dist2(pos, lp.pos);
-            double pdf_nee = S.light_pmf[lid] * pdf_shape<SPH>(S.shapes[l.shape_id], lp, pos);
+            double pdf_nee = S.light_pmf[lid] * pdf_light_point<SPH, ENV>(S, l, lp, pos);
             if (G > 0 && pdf_nee > 0) {
                 D3 f;
                 double pdf_f;
@@ -392,7 +392,7 @@ __device__ __forceinline__ void vol_shade(const DeviceScene &S, const PathBufs &
                     f = bsdf_eval<DMT>(mat, dir_view, dir_light, v.g);
                     pdf_f = bsdf_pdf<DMT>(mat, dir_view, dir_light, v.g);
                 }
-                D3 L = light_emission(l, -dir_light, lp);
+                D3 L = light_emission<ENV>(l, -dir_light, lp);
                 D3 K = pre * G * f * L;
                 if (K.x != 0 || K.y != 0 || K.z != 0) {
                     push_sh = true;
@@ -446,12 +446,12 @@ __device__ __forceinline__ void vol_shade(const DeviceScene &S, const PathBufs &
     }
 }
 
-// Surfaces: DMT is the material type of the kernel's bucket, or -1 for the
-// buckets from kVolTyped on.
+// Surfaces: DMT is the material type of the kernel's bucket, -1 for the
+// buckets from kVolTyped on, or kMtEnv for all of them.
 constexpr int kVolTyped = 3;
 template <bool SPH, int DMT, int EV>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EV == kEvSurface && DMT >= 0 && !SPH ? 2 : 1))) void k_vol_shade(DeviceScene S, PathBufs P, int cur) {
-    constexpr int first = EV == kEvScatter ? kBucketScatter : EV == kEvPass ? kBucketNoMat : DMT >= 0 ? DMT : kVolTyped;
+    constexpr int first = EV == kEvScatter ? kBucketScatter : EV == kEvPass ? kBucketNoMat : DMT >= 0 ? DMT : DMT == kMtEnv ? 0 : kVolTyped;
     constexpr int end = EV == kEvSurface && DMT < 0 ? kBucketScatter : first + 1;
     const int j0 = bucket_start(P, first), j1 = bucket_start(P, end);
     for (int j = j0 + blockIdx.x * blockDim.x + threadIdx.x; j < j1; j += gridDim.x * blockDim.x) {
@@ -776,7 +776,9 @@ inline void vol_events(const DeviceScene &S, PathBufs &P, int cur, int grid, hip
     vol_launch_check();
 }
 // The shading kernels, on the streams given (one may stand for all three).
-// types: the material types present; textured: some material reads a texture.
+// types: the material types present; textured: some material reads a texture;
+// env: an envmap is among the lights (the kernels for spheres take scenes
+// without them too).
 template <bool SPH>
 void vol_shade_t(const DeviceScene &S, PathBufs &P, int cur, int grid, const hipStream_t (&s)[3], unsigned types,
                  bool textured) {
@@ -791,8 +793,14 @@ void vol_shade_t(const DeviceScene &S, PathBufs &P, int cur, int grid, const hip
     vol_launch_check();
 }
 inline void vol_shade_all(const DeviceScene &S, PathBufs &P, int cur, int grid, const hipStream_t (&s)[3], bool sph,
-                          unsigned types, bool textured) {
-    if (sph) vol_shade_t<true>(S, P, cur, grid, s, types, textured);
+                          unsigned types, bool textured, bool env) {
+    if (env) {
+        const dim3 g(grid), b(256);
+        hipLaunchKernelGGL((k_vol_shade<true, kMtEnv, kEvSurface>), g, b, 0, s[0], S, P, cur);
+        hipLaunchKernelGGL((k_vol_shade<true, kMtEnv, kEvScatter>), g, b, 0, s[1], S, P, cur);
+        hipLaunchKernelGGL((k_vol_shade<true, kMtEnv, kEvPass>), g, b, 0, s[2], S, P, cur);
+        vol_launch_check();
+    } else if (sph) vol_shade_t<true>(S, P, cur, grid, s, types, textured);
     else vol_shade_t<false>(S, P, cur, grid, s, types, textured);
 }
 
