@@ -35,12 +35,13 @@ constexpr int kNumBuckets = 13;
 // counter slots
 constexpr int C_EXT = 0;      // C_EXT + (0|1): extension queues
 constexpr int C_BUCKET = 4;   // C_BUCKET + bucket: its paths
-constexpr int C_TOTAL = 16;
+constexpr int C_HOST = C_BUCKET + kNumBuckets;  // the counters the host reads back
 // ticket counters (Feed), in sets of kFeeds a 128-byte line apart: two for
 // the closest-hit launches, used in turn by the bounces, and one each for the
 // bounce's other launches
 constexpr int kFeeds = 8, kFeedLine = 32, kFeedSet = kFeeds * kFeedLine;
 constexpr int C_FEED = 32;
+static_assert(C_HOST <= C_FEED && C_FEED % kFeedLine == 0, "queue counters share no line with tickets");
 constexpr int C_FEED_SHADOW = C_FEED + 2 * kFeedSet;
 constexpr int C_FEED_WALK = C_FEED + 3 * kFeedSet;
 constexpr int C_FEED_FLIGHT = C_FEED + 4 * kFeedSet;

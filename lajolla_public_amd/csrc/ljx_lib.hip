@@ -1363,7 +1363,7 @@ void render_impl(Scene &sc, const ljx_render_options *o, const ljx_exec_options 
 
     uint64_t passes = 0, train_samples = 0, train_steps = 0, train_step_samples = 0;
     int max_bounces = opt.max_depth >= 0 ? std::max(opt.max_depth, 1) : 1 << 20;
-    std::vector<int> host_ctr(C_TOTAL);
+    std::vector<int> host_ctr(C_HOST);
     const int train_spp = guided ? std::min(gopt.train_spp, spp) : 0;
     for (int s0 = 0; s0 < spp;) {
         const bool recording = s0 < train_spp;
@@ -1393,7 +1393,7 @@ void render_impl(Scene &sc, const ljx_render_options *o, const ljx_exec_options 
             for (int b = 0; b < max_bounces; b++) {
                 if (opt.max_depth < 0 && b >= 8) {
                     // RR-only paths: stop once the extension queue drains
-                    HIPX(hipMemcpyAsync(host_ctr.data(), P.ctr, sizeof(int) * C_TOTAL, hipMemcpyDeviceToHost, s));
+                    HIPX(hipMemcpyAsync(host_ctr.data(), P.ctr, sizeof(int) * C_HOST, hipMemcpyDeviceToHost, s));
                     HIPX(hipStreamSynchronize(s));
                     if (host_ctr[C_EXT + cur] == 0) break;
                 }
