@@ -21,6 +21,7 @@
 // shape or queue order.
 #pragma once
 
+#include "ljx_feed.h"
 #include "ljx_guide.h"
 #include "ljx_shade.h"
 
@@ -36,10 +37,8 @@ constexpr int kNumBuckets = 13;
 constexpr int C_EXT = 0;      // C_EXT + (0|1): extension queues
 constexpr int C_BUCKET = 4;   // C_BUCKET + bucket: its paths
 constexpr int C_HOST = C_BUCKET + kNumBuckets;  // the counters the host reads back
-// ticket counters (Feed), in sets of kFeeds a 128-byte line apart: two for
-// the closest-hit launches, used in turn by the bounces, and one each for the
-// bounce's other launches
-constexpr int kFeeds = 8, kFeedLine = 32, kFeedSet = kFeeds * kFeedLine;
+// ticket counters (Feed), in sets: two for the closest-hit launches, used in
+// turn by the bounces, and one each for the bounce's other launches
 constexpr int C_FEED = 32;
 static_assert(C_HOST <= C_FEED && C_FEED % kFeedLine == 0, "queue counters share no line with tickets");
 constexpr int C_FEED_SHADOW = C_FEED + 2 * kFeedSet;
@@ -418,59 +417,6 @@ __global__ void k_raygen(DeviceScene S, PathBufs P) {
     }
 }
 
-// Hands a launch's n queue entries to its waves, 64 at a time, so that waves
-// that drew short work take more and the launch's tail stays short.  Each
-// wave's first chunk is its own by its number; after that it takes tickets.
-// A ticket is one atomic by the whole wave, and those on one cache line run
-// one every 11.3 ns on the whole chip (2,048 blocks took 12 ms of tickets for
-// 67M rays from a single counter), so blocks draw from kFeeds counters on
-// lines of their own, by block number modulo kFeeds, which is the XCD that
-// dispatch in turn places them on.  Feed f owns every kFeeds-th run of
-// kFeedRun chunks: an XCD's waves work on neighbouring entries, and every feed
-// sees all parts of the queue.
-constexpr int kFeedRun = 16;
-// A ticket's round trip takes over a microsecond, which two or three waves per
-// SIMD do not hide.  For kernels of such occupancy a ticket covers several
-// chunks of a long queue, as many as leave every wave `tickets` of them (media
-// render's shadow walks 14.9 -> 7.5 ms); at eight waves per SIMD single chunks
-// are better (terrain's closest hits 56.4 against 58.8 ms).
-constexpr int kFeedTickets = 8;
-struct Feed {
-    int feeds, feed, waves, ticket, sub, span;
-    int *counter;
-    bool more;  // tickets remain after every wave's first
-    __device__ __forceinline__ int chunk(int t) const {
-        return ((t * span / kFeedRun) * feeds + feed) * kFeedRun + t * span % kFeedRun;
-    }
-    // counters: a set of kFeeds zeroed counters kFeedLine apart.  Grids of
-    // fewer than kFeeds blocks use one feed.
-    __device__ __forceinline__ void start(int *counters, int n, int tickets = 0) {
-        const int wpb = blockDim.x >> 6, chunks = (n + 63) / 64;
-        feeds = int(gridDim.x) < kFeeds ? 1 : kFeeds;
-        feed = int(blockIdx.x) % feeds;
-        waves = (int(gridDim.x) + feeds - 1 - feed) / feeds * wpb;
-        span = 1;
-        while (tickets > 0 && span < kFeedRun && chunks >= 2 * span * tickets * int(gridDim.x) * wpb) span *= 2;
-        ticket = __builtin_amdgcn_readfirstlane(int(blockIdx.x) / feeds * wpb + int(threadIdx.x >> 6));
-        sub = 0;
-        counter = counters + feed * kFeedLine;
-        more = chunk(waves) < chunks;
-    }
-    // First entry of the wave's current chunk; at or past n: none is left.
-    __device__ __forceinline__ int base() const { return (chunk(ticket) + sub) * 64; }
-    __device__ __forceinline__ void next(int n) {
-        if (++sub < span) return;
-        sub = 0;
-        if (!more) {
-            ticket = (1 << 20) / span;  // past every queue (2^26 entries)
-            return;
-        }
-        int t = 0;
-        if (__lane_id() == 0) t = atomicAdd(counter, 1);
-        ticket = waves + __builtin_amdgcn_readfirstlane(t);
-    }
-};
-
 // Closest-hit traversal of the extension queue: a wave walks 64 rays (Feed)
 // until the last one ends; each hit's distance is refined while its triangle
 // is in cache, and each queue entry gets the key of the material it hit.
@@ -527,7 +473,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH ? 1 : 8
     uint32_t nn = 0, np = 0;
     Feed feed;
     feed.start(feeds + cur * kFeedSet, n);
-    for (int base = feed.base(); base < n; feed.next(n), base = feed.base()) {
+    for (int base = feed.base(); base < n; feed.next(), base = feed.base()) {
         const int i = base + lane;
         if (i < n) {
             const uint32_t pid = q[i];
@@ -834,7 +780,7 @@ struct FeedRange {
         };
         while (w && !done) {
             if (at == count) {
-                if (!fresh) feed.next(n);
+                if (!fresh) feed.next();
                 fresh = false;
                 const int base = feed.base();
                 if (base >= n) {
