@@ -167,3 +167,23 @@ def test_grey_media_kernels_equal_the_general_ones(res):
     assert a.mean() > 0
     # a path whose real-or-null draw falls between the two roundings would part: none of some 10^5 draws at 1e-15 each
     assert np.allclose(a, b, rtol=1e-5, atol=1e-8)
+
+
+@pytest.mark.parametrize("grey", [True, False])
+def test_flights_and_walks_by_tickets_of_several_chunks(grey):
+    """On a queue long for its grid a ticket of the flight and walk kernels covers several chunks of it: 17.7M paths
+    in one pass give the flights' 16,384 waves two chunks a ticket and, at one block per CU, the walks' 1,024 waves
+    sixteen.  The same render in passes too short for more than one chunk a ticket takes the same samples."""
+    desc = scenes.hetvol_smoke(seed=3, res=32, scale=40.0, width=768, height=576, spp=40, max_depth=3)
+    if not grey:
+        desc.add_medium((0.1, 0.2, 0.3), (0.3, 0.2, 0.1))
+    sc = api.Scene(desc)
+    opts = scenes.render_options(**desc.options)
+    img, st = sc.render(options=opts, stats=True,
+                        exec_options=api.exec_options(trace_blocks_per_cu=1, max_paths_in_flight=1 << 25))
+    part, sp = sc.render(options=opts, stats=True, exec_options=api.exec_options(max_paths_in_flight=1 << 19))
+    assert (st["passes"], sp["passes"] > 1) == (1, True)
+    for k in ("camera_paths", "extension_rays", "shadow_rays"):
+        assert st[k] == sp[k], k
+    # a pixel's samples added in other groups in FP64, rounded once to FP32
+    assert img.mean() > 0 and np.allclose(img, part, rtol=2e-6, atol=1e-9)

@@ -138,10 +138,10 @@ def test_analytic_glass_sphere():
 
 @pytest.mark.parametrize("mat", ["basic", "disney"])
 def test_volpath_material_dispatch_sample_matched(mat):
-    """Volumetric shading dispatches BSDFs over lajolla's three basic
-    materials only when the scene uses no others, else over every type:
-    the nested-media scene as it is (Lambertian, RoughDielectric) and with
-    its floor made DisneyBSDF, both sample-matched to the oracle."""
+    """Surface hits of volumetric paths: the nested-media scene as it is
+    (Lambertian and RoughDielectric, each shaded by its own kernel) and with
+    its floor made DisneyBSDF (the run-time-dispatch kernel), both
+    sample-matched to the oracle."""
     desc = scenes.nested_media(seed=11, g=0.7, width=40, height=40, spp=8, max_depth=10, sphere_res=32)
     if mat == "disney":
         floor = [s for s in desc.shapes if s["positions"].shape[0] == 4 and s["positions"][:, 1].max() == 0.0][0]
@@ -152,3 +152,34 @@ def test_volpath_material_dispatch_sample_matched(mat):
     assert np.isfinite(g).all()
     sample_matched(g, o, frac=0.90)
     assert abs(g.mean() - o.mean()) < 0.03 * o.mean()
+
+
+@pytest.mark.parametrize("spheres", [False, True])
+def test_volpath_every_bucket_sample_matched(spheres):
+    """Every bucket of volumetric surface hits at once: the three basic
+    materials, shaded by a kernel each, the other types and a textured
+    material, whose adjoining buckets one run-time-dispatch kernel spans,
+    pass-through boundaries, scattering and misses."""
+    desc = scenes.nested_media(seed=11, g=0.7, width=48, height=48, spp=8, max_depth=8, sphere_res=24)
+    mats = [desc.add_material(t, (0.7, 0.5, 0.4), (0.6, 0.7, 0.8), roughness=0.3, eta=1.5, specular=0.5,
+                              sheen_tint=0.3, clearcoat_gloss=0.7, metallic=0.4, clearcoat=0.5, sheen=0.4)
+            for t in range(9)]
+    chk = desc.add_checkerboard((0.8, 0.7, 0.6), (0.1, 0.2, 0.3), uscale=4, vscale=4)
+    mats.append(desc.add_material(capi.MAT_ROUGH_PLASTIC, (0, 0, 0), (0.5, 0.5, 0.5), roughness=0.2,
+                                  textures={"color_a": chk}))
+    for k, m in enumerate(mats):
+        x, z = -2.2 + 1.1 * (k % 5), 1.3 + 0.9 * (k // 5)
+        if spheres and k % 2:
+            desc.add_sphere((x, 0.4, z), 0.35, m)
+        else:
+            P, I, N = scenes.box((x, 0.4, z), (0.6, 0.6, 0.6), 20.0 * k)
+            desc.add_mesh(P, I, m, normals=N, uvs=np.tile([[0, 0], [1, 0], [1, 1], [0, 1]], (len(P) // 4, 1)))
+    sc = api.Scene(desc)
+    g, st = sc.render(stats=True)
+    o, _ = po.OracleScene(desc).render(plan=1)
+    assert np.isfinite(g).all()
+    sample_matched(g, o, frac=0.90)
+    assert abs(g.mean() - o.mean()) < 0.03 * o.mean()
+    # smaller passes leave some buckets empty
+    part = sc.render(options=scenes.render_options(**desc.options), exec_options=api.exec_options(max_paths_in_flight=640))
+    assert np.allclose(g, part, rtol=2e-6, atol=1e-9)
