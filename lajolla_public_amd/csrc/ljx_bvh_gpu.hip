@@ -42,8 +42,10 @@ constexpr int kChunk = 2048;  // primitives per block in the wide-range kernels
 // wave's boxes and bins take 19 KB of LDS, two waves per SIMD, and a wave
 // hides nothing of its serial steps; at 256 it is 11 KB and three to four: the
 // narrow ranges of 2.3M triangles 11.5 -> 8.9 ms for 0.5 ms more of wide
-// levels, opening the scene 43.5 -> 41.1 ms.  At 128 the wide levels grow by
-// 1.4 ms and their bins to 48 MB: 42.1 ms.
+// levels, opening the scene 43.3 -> 41.3 ms (six runs of each in turn, their
+// ranges apart), one of 512 triangles 3.8 -> 2.4 ms.  At 128 the narrow ranges
+// take 8.0 ms, but the wide levels 1.5 ms more than at 512 and 48 MB of bins:
+// 41.7 ms.
 constexpr int kSmall = 256;
 constexpr int kWaveStack = 32;
 constexpr int kBinInts = 3 * kBvhBins * 7;  // per bin: count, lo xyz, hi xyz

@@ -98,7 +98,7 @@ struct PathBufs {
     int pass_s0, pass_ns, pass_q0, pass_nq;
     int spp, max_depth, rr_depth;
     int volpath;
-    int vol_flight;  // free flight runs in k_vol_flight (scenes with grid media), else inside k_vol_shade
+    int vol_flight;  // free flight runs in k_vol_flight (scenes with grid media), else in k_vol_event and k_vol_shade
     int vol_grey;    // every medium is a grid of one density channel
     int max_null;
     uint64_t seed;
@@ -691,17 +691,18 @@ __device__ __forceinline__ void shade_queue(const DeviceScene &S, const PathBufs
     }
 }
 
-// The shading kernel of one material type (or, MT < 0, of run-time dispatch).  Occupancy of these FP64-heavy kernels is set by their register
-// count: 185-204 for Lambertian, RoughPlastic, DisneyDiffuse, DisneyMetal and
-// DisneySheen without spheres in the scene, under 257 with them, hence two
-// waves per SIMD; DisneyBSDF spills at two, but running beside the other
-// types' kernels is faster there than at one (shading of the 1080p large-mesh
-// render 42.1 -> 40.6 ms).  Three waves, which the first five reach with
+// The shading kernel of one material type (or, MT < 0, of run-time dispatch).
+// Occupancy of these FP64-heavy kernels is set by their register count:
+// 185-204 for Lambertian, RoughPlastic, DisneyDiffuse, DisneyMetal and
+// DisneySheen without spheres in the scene, 255 or 256 with them (up to 22
+// spilled), hence two waves per SIMD; DisneyBSDF spills at two, but running
+// beside the other types' kernels is faster there than at one (shading of the
+// 1080p large-mesh render 42.1 -> 40.6 ms).  Three waves, which the first five reach with
 // little spilling, are slower, 43.0 against 35.4 ms for the same shading: the
 // kernels keep the vector-memory data unit 0.9 busy, and more waves beside
 // DisneyBSDF's only take its share of it.
-// RoughDielectric, DisneyGlass and DisneyClearcoat need four registers more
-// than two waves allow without spheres, and too many with them.
+// RoughDielectric, DisneyGlass and DisneyClearcoat fit two waves without
+// spheres (241-254 registers) and keep one with them (304-322).
 constexpr int shade_waves(int mt, bool sph) { return mt < 0 || (sph && (mt == 2 || mt == 5 || mt == 6)) ? 1 : 2; }
 template <int MT, bool SPH, bool GUIDE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(shade_waves(MT, SPH)))) void k_shade(

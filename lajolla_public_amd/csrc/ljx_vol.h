@@ -107,8 +107,9 @@ __device__ __forceinline__ void flight_begin(FlightRun &r, const DeviceScene &S,
 // the three channels stay equal and only the first is computed (x); majorant
 // over largest majorant, one there, drops out.  A third of the FP64 lookups,
 // divisions and state: the 128^3 smoke grid's flights and walks are bound by
-// that arithmetic and by the two waves per SIMD its registers allow (71 -> 37
-// and 87 -> 45 ms at 768x576, 64 samples, at four and three waves).
+// that arithmetic and by the waves per SIMD its registers allow (71 -> 37 and
+// 87 -> 45 ms at 768x576, 64 samples, at four waves instead of three and three
+// instead of two).
 // One pass of the loop; true when the flight has ended.  decided: whether the
 // path collides before its hit, where an earlier kernel has found that out (1
 // or 0, else -1): two compilations of the comparison may round differently.
@@ -215,10 +216,10 @@ __global__ __launch_bounds__(256) void k_vol_event(DeviceScene S, PathBufs P, in
 }
 
 // Free flight for the queue's paths that are in a medium, in a kernel small
-// enough for three waves per SIMD.  The loops' lengths vary widely between
-// paths, so a lane whose flight ended (or whose path is in no medium) takes
-// its next path as soon as kFlightRefill lanes of its wave are idle rather
-// than waiting for the wave's longest flight.
+// enough for three waves per SIMD (GREY: four).  The loops' lengths vary
+// widely between paths, so a lane whose flight ended (or whose path is in no
+// medium) takes its next path as soon as kFlightRefill lanes of its wave are
+// idle rather than waiting for the wave's longest flight.
 constexpr int kFlightRefill = 16;
 template <bool SPH, bool GREY>
 __global__ __launch_bounds__(256) void k_vol_flight(DeviceScene S, PathBufs P, int cur) {
