@@ -1151,7 +1151,7 @@ void trace_stage_t(Scene &sc, PathBufs &P, int cur, int grid, int sgrid, hipStre
 // path id can name (67,108,864).  Traversal and shading launches need many
 // rays per lane to amortise their tails: a 1080p render runs at 359, 639, 693
 // and 723 Msamples/s with 4M, 16M, 32M and 64M paths per pass.  The path
-// state is ~0.5 KB per path (31 GB for a 1080p pass of 32 samples per pixel).
+// state is 287 B per path (19 GB for a 1080p pass of 32 samples per pixel).
 constexpr int kDefaultPathsInFlight = 1 << kSlotBits;
 
 // The next extension queue from the flags shading left (k_alive_*).
